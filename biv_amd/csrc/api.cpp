@@ -328,11 +328,11 @@ int dense_scratch_fit(biv_hip_ctx *ctx, const biv_hip_dense *d, int T)
     const size_t Tc = cap;
     auto *b = &s.bufs;
     int rc = 0;
-    rc = rc ? rc : sc_alloc(ctx, Tc * E, &s.xq, b);
+    rc = rc ? rc : sc_alloc(ctx, Tc * E * 2, &s.xq, b); // int8 or f16 quants
     rc = rc ? rc : sc_alloc(ctx, Tc * E / 32, &s.xd, b);
     rc = rc ? rc : sc_alloc(ctx, Tc * E / 32, &s.xs, b);
     rc = rc ? rc : sc_alloc(ctx, Tc * ff, &s.act, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * ff, &s.aq, b);
+    rc = rc ? rc : sc_alloc(ctx, Tc * ff * 2, &s.aq, b);
     rc = rc ? rc : sc_alloc(ctx, Tc * ff / 32, &s.ad, b);
     rc = rc ? rc : sc_alloc(ctx, Tc * ff / 32, &s.as, b);
     rc = rc ? rc : sc_alloc(ctx, Tc * E, &s.h_stage, b);
@@ -347,6 +347,20 @@ int dense_scratch_fit(biv_hip_ctx *ctx, const biv_hip_dense *d, int T)
     return 0;
 }
 
+// Whether a half of the dense FFN (T rows against a matrix of rows x K) runs
+// on the matrix cores (launch_exact) or in the chain matvecs (launch_long_mv).
+// The matvecs' time grows with the tokens, the matrix-core kernel's up to 16
+// tokens is the latency of its K steps: layers of 4096 x 12288 cross between
+// 5 and 6 tokens (Q8_0 at 6 / 8 / 16: 87 / 88 / 93 against 90 / 105 / 150 us;
+// Q4_K/Q6_K at 5 / 8 / 16: 101 / 102 / 108 against 118 / 186 / 318), small
+// Q8_0 layers later (1024 x 1536 at 20 / 40: 27 / 27 against 22 / 29; 2048 x
+// 3584 at 8 / 12: 31 / 32 against 30 / 34; 1536 x 7680 at 7: 43 against 44).
+bool dense_exact(int ty, int T, int rows, int K)
+{
+    if (ty == biv::T_BF16 || T < 7) return false;
+    return ty != biv::T_Q8_0 || (size_t)T * rows * K >= ((size_t)72 << 20);
+}
+
 // dense_ffn (model.rs:1118-1126) of T rows on the context's stream:
 // Input::q8 of h (for quantised gate/up), gate/up with the SwiGLU, Q8 of
 // the intermediate (for a quantised down), down into out or added to it.
@@ -359,33 +373,43 @@ int dense_forward(biv_hip_ctx *ctx, const biv_hip_dense *d, const float *h, int 
     hipStream_t st = ctx->stream;
     const int E = d->E, ff = d->ff;
     const DevMat &G = d->gate->m, &U = d->up->m, &D = d->down->m;
-    if (G.ty != biv::T_BF16)
-        HIP_TRY(ctx, biv::launch_quant_rows(h, T * E / 32, E, s.xq, s.xd, s.xs, st), "quantise h");
-    biv::LongArgs g{};
-    g.a = G;
-    g.b = U;
-    g.xq = s.xq;
-    g.xd = s.xd;
-    g.xs = s.xs;
-    g.xf = h;
-    g.out = s.act;
-    g.T = T;
-    g.K = E;
-    HIP_TRY(ctx, biv::launch_long_mv(g, 1, st), "dense gate/up");
-    if (D.ty != biv::T_BF16)
-        HIP_TRY(ctx, biv::launch_quant_rows(s.act, T * ff / 32, ff, s.aq, s.ad, s.as, st), "quantise act");
-    biv::LongArgs dn{};
-    dn.a = D;
-    dn.xq = s.aq;
-    dn.xd = s.ad;
-    dn.xs = s.as;
-    dn.xf = s.act;
-    dn.out = out;
-    dn.T = T;
-    dn.K = ff;
-    dn.add = (flags & BIV_HIP_ADD) != 0;
-    HIP_TRY(ctx, biv::launch_long_mv(dn, 0, st), "dense down");
-    return 0;
+    // one half of the layer: the input rows quantised (unless BF16), then
+    // the product
+    auto half = [&](const DevMat &A, const DevMat *B, const float *in, int K, int8_t *q, float *qd, float *qs,
+                    float *dst, int add, const char *what) -> int {
+        const int n_blocks = T * (K / 32);
+        if (dense_exact(A.ty, T, A.rows, K)) {
+            biv::ExactArgs e{};
+            e.a = A;
+            if (B) e.b = *B;
+            e.xh = reinterpret_cast<const uint16_t *>(q);
+            e.xd = qd;
+            e.xs = qs;
+            e.out = dst;
+            e.T = T;
+            e.K = K;
+            e.add = add;
+            HIP_TRY(ctx, biv::launch_quant_f16(in, n_blocks, reinterpret_cast<uint16_t *>(q), qd, qs, st), "quantise");
+            HIP_TRY(ctx, biv::launch_exact(e, B != nullptr, st), what);
+            return 0;
+        }
+        if (A.ty != biv::T_BF16) HIP_TRY(ctx, biv::launch_quant_rows(in, n_blocks, K, q, qd, qs, st), "quantise");
+        biv::LongArgs g{};
+        g.a = A;
+        if (B) g.b = *B;
+        g.xq = q;
+        g.xd = qd;
+        g.xs = qs;
+        g.xf = in;
+        g.out = dst;
+        g.T = T;
+        g.K = K;
+        g.add = add;
+        HIP_TRY(ctx, biv::launch_long_mv(g, B != nullptr, st), what);
+        return 0;
+    };
+    if ((rc = half(G, &U, h, E, s.xq, s.xd, s.xs, s.act, 0, "dense gate/up"))) return rc;
+    return half(D, nullptr, s.act, ff, s.aq, s.ad, s.as, out, (flags & BIV_HIP_ADD) != 0, "dense down");
 }
 
 void scratch_free(biv_hip_ctx *ctx)

@@ -168,6 +168,22 @@ struct LongArgs {
 };
 hipError_t launch_long_mv(const LongArgs &a, int gateup, hipStream_t st);
 
+// The same contract over many tokens on the matrix cores (exact.hip), for
+// quantised matrices: the chain kernels' bits.  The activations are the Q8
+// quants as f16 (launch_quant_f16's order), with their block scales and sums
+// in block order.
+struct ExactArgs {
+    DevMat a, b;           // gate and up (b), or down (a)
+    const uint16_t *xh;    // [T][K] f16
+    const float *xd, *xs;  // [T][K / 32]
+    float *out;            // [T][rows]
+    int T, K, add;
+};
+hipError_t launch_exact(const ExactArgs &a, int gateup, hipStream_t st);
+// Q8Act of n_blocks 32-element blocks, in element order but for the 8 words
+// (of four quants) of a block, which go 0, 4, 1, 5, 2, 6, 3, 7
+hipError_t launch_quant_f16(const float *x, int n_blocks, uint16_t *xh, float *d, float *s, hipStream_t st);
+
 // BF16 experts at prefill sizes on the matrix cores (mfma.hip).  The input
 // rows are first split into bf16 hi / lo halves (launch_split_bf16); gate/up
 // writes the f32 SwiGLU intermediate, down the f32 y rows, as the chain

@@ -11,14 +11,13 @@
 #include "expf_ref.h"
 #include "layout.hpp"
 #include "lds_dma.hpp"
+#include "mfma_ops.hpp"
 
 #include <hip/hip_fp16.h>
 
 namespace biv {
 
 namespace {
-
-constexpr int WAVE = 64;
 
 __device__ inline int dot4(int a, int b, int c) { return __builtin_amdgcn_sdot4(a, b, c, false); }
 
@@ -77,10 +76,11 @@ template <int N> __device__ inline void ld_words(const void *p, int (&out)[N])
 // Q8Act::quantize_into (quant.rs:368-394) of one 32-element block v of row
 // `row`: amax, d = amax / 127, id = 1/d (0 when d is 0), q =
 // round-half-away(v * id), s = d * sum(q); IEEE division and no contraction
-// keep it bit-exact.  Written in the chain layout (layout.hpp).
+// keep it bit-exact (quant_words: the quants as bytes).  quant_block_at
+// writes it in the chain layout (layout.hpp).
 // The row's quant words, block scales and block sums are at qrow, drow, srow
 // (srow may be null); generic pointers, so the row may be in LDS.
-__device__ inline void quant_block_at(const float (&v)[32], int K, int b, int *qrow, float *drow, float *srow)
+__device__ inline void quant_words(const float (&v)[32], unsigned (&q)[8], float &d, float &s)
 {
     // the largest magnitude as a tree: max is exact, so any order gives the
     // sequential loop's value (NaNs skipped by fmaxf alike; 0 if all are)
@@ -104,10 +104,20 @@ __device__ inline void quant_block_at(const float (&v)[32], int K, int b, int *q
             sum += r;
             w |= (unsigned)(r & 0xFF) << (8 * c);
         }
-        qrow[lay::q8_word(b, l)] = (int)w;
+        q[l] = w;
     }
-    drow[lay::q8_scale(K, b)] = db;
-    if (srow) srow[lay::q8_scale(K, b)] = db * (float)sum;
+    d = db;
+    s = db * (float)sum;
+}
+__device__ inline void quant_block_at(const float (&v)[32], int K, int b, int *qrow, float *drow, float *srow)
+{
+    unsigned q[8];
+    float d, s;
+    quant_words(v, q, d, s);
+#pragma unroll
+    for (int l = 0; l < 8; l++) qrow[lay::q8_word(b, l)] = (int)q[l];
+    drow[lay::q8_scale(K, b)] = d;
+    if (srow) srow[lay::q8_scale(K, b)] = s;
 }
 
 // The same from a block in LDS, read twice (amax, then the quants) so that
@@ -2464,6 +2474,25 @@ __global__ __launch_bounds__(256) void k_quant_rows(const float *__restrict__ x,
     quant_block(v, K, i / (K / 32), i % (K / 32), qs, d, s);
 }
 
+// The same with the quants as f16, words l and l + 4 of a block (four quants
+// each) side by side, and the blocks in element order (exact.hip).
+__global__ __launch_bounds__(256) void k_quant_f16(const float *__restrict__ x, int n_blocks, uint16_t *__restrict__ xh,
+                                                   float *__restrict__ d, float *__restrict__ s)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_blocks) return;
+    float v[32];
+    load32(x + 32 * (size_t)i, v);
+    unsigned q[8];
+    quant_words(v, q, d[i], s[i]);
+    uint4 *o = reinterpret_cast<uint4 *>(xh + 32 * (size_t)i);
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+        const uint2 a = i8x4_to_f16x4(q[l]), b = i8x4_to_f16x4(q[l + 4]);
+        o[l] = make_uint4(a.x, a.y, b.x, b.y);
+    }
+}
+
 // The combine as its own launch: grid (E / 256, T).
 __global__ __launch_bounds__(256) void k_combine(CombineArgs a)
 {
@@ -2886,6 +2915,13 @@ hipError_t launch_quant_rows(const float *x, int n_blocks, int K, int8_t *qs, fl
 {
     if (n_blocks <= 0) return hipSuccess;
     k_quant_rows<<<(n_blocks + 255) / 256, 256, 0, st>>>(x, n_blocks, K, qs, d, s);
+    return hipGetLastError();
+}
+
+hipError_t launch_quant_f16(const float *x, int n_blocks, uint16_t *xh, float *d, float *s, hipStream_t st)
+{
+    if (n_blocks <= 0) return hipSuccess;
+    k_quant_f16<<<(n_blocks + 255) / 256, 256, 0, st>>>(x, n_blocks, xh, d, s);
     return hipGetLastError();
 }
 

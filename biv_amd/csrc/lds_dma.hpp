@@ -27,6 +27,20 @@ __device__ inline void lds_dma16_at(const void *g, unsigned lds_addr)
     const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_addr);
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(m0) : "memory", "m0");
 }
+// The same from a uniform base and a 32-bit byte offset per lane, 16 bytes or
+// one dword (LDS address m0 + 4 lane) a lane.
+__device__ inline void lds_dma16_off(const void *base, uint32_t off, unsigned lds_addr)
+{
+    const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_addr);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0)
+                 : "memory", "m0");
+}
+__device__ inline void lds_dma4_off(const void *base, uint32_t off, unsigned lds_addr)
+{
+    const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_addr);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0)
+                 : "memory", "m0");
+}
 // the LDS address (byte offset) of a shared-memory pointer
 __device__ inline unsigned lds_addr(const void *p)
 {

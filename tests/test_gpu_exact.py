@@ -1,0 +1,85 @@
+"""The matrix-core kernel of the dense FFN (k_exact) against the oracle's
+dense_ffn: every output carries the oracle's bits, at the edges of its tiles
+(16, 32 and 64 input rows a workgroup, a last workgroup that holds fewer),
+for every quantised type, from one chunk pair of a row up.  Its operations
+and their order are the reference's, so the bound is equality."""
+import numpy as np
+import pytest
+
+from biv_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+Q8_0, Q4K, Q6K, BF16 = synth.Q8_0, synth.Q4K, synth.Q6K, synth.BF16
+
+
+@pytest.fixture(scope="module")
+def engine():
+    from biv_amd import hip
+    e = hip.HipEngine(0)
+    yield e
+    e.close()
+
+
+def run(orc, engine, types, n_embd, n_ff, tokens, edit=None):
+    layer = synth.make_dense(21, n_embd=n_embd, n_ff=n_ff, types=types)
+    d = engine.dense(layer)
+    g, u, dn = layer.gate, layer.up, layer.down
+    for T in tokens:
+        print(f"case {types} {n_embd} x {n_ff} T={T}", flush=True)
+        h = synth.make_tokens(1000 + T, T, n_embd=n_embd)
+        if edit:
+            edit(h)
+        ref = orc.dense_ffn(g.ty, g.data, u.ty, u.data, dn.ty, dn.data, n_embd, n_ff, h, threads=8)
+        got = d.ffn(h)
+        same = ref.view(np.uint32) == got.view(np.uint32)
+        assert np.all(same | (np.isnan(ref) & np.isnan(got))), f"{np.mean(~same):.2e} of the outputs differ"
+        x = synth.make_tokens(2000 + T, T, n_embd=n_embd)
+        add = d.ffn(h, out=x.copy(), add=True)
+        assert np.array_equal(add, x + ref, equal_nan=True)
+
+
+# 16-row tiles (and the smallest rows, where Q8_0 takes the matvecs)
+@pytest.mark.parametrize("types,n_embd,n_ff,tokens", [
+    ((Q8_0, Q8_0, Q8_0), 2048, 2560, (15, 16)),
+    ((Q4K, Q4K, Q6K), 1536, 2560, (7, 16)),
+    ((Q6K, Q6K, Q4K), 512, 512, (7, 15, 16)),
+    ((Q4K, Q4K, BF16), 512, 1024, (9,)),
+    ((BF16, BF16, Q6K), 1024, 512, (9,)),
+])
+def test_exact_16(orc, engine, types, n_embd, n_ff, tokens):
+    run(orc, engine, types, n_embd, n_ff, tokens)
+
+
+@pytest.mark.parametrize("types,n_embd,n_ff,tokens", [
+    ((Q8_0, Q8_0, Q8_0), 2048, 2560, (17, 32, 33, 48, 65)),
+    ((Q8_0, Q8_0, Q8_0), 512, 2048, (73, 129)),
+    ((Q4K, Q4K, Q6K), 1536, 2560, (17, 32, 33, 64)),
+    ((Q6K, Q6K, Q4K), 512, 512, (17, 33, 50)),
+])
+def test_exact_32(orc, engine, types, n_embd, n_ff, tokens):
+    run(orc, engine, types, n_embd, n_ff, tokens)
+
+
+# enough output rows for 64-row tiles: the last of 36 (three tiles), 64, 8 and 32 rows
+@pytest.mark.parametrize("types", [(Q8_0, Q8_0, Q8_0), (Q4K, Q4K, Q6K), (Q6K, Q6K, Q4K)])
+@pytest.mark.parametrize("n_embd,n_ff,tokens", [(512, 16384, (100, 128, 200, 224)), (16384, 512, (100, 128))])
+def test_exact_64(orc, engine, types, n_embd, n_ff, tokens):
+    run(orc, engine, types, n_embd, n_ff, tokens)
+
+
+@pytest.mark.parametrize("types,T", [((Q8_0, Q8_0, Q8_0), 40), ((Q4K, Q4K, Q6K), 20)])
+def test_exact_special_rows(orc, engine, types, T):
+    """Rows of zeros, of huge and tiny values, and with an infinity or a NaN,
+    beside ordinary ones.  (Q4_K's mins read the block sums, and the oracle
+    sums a NaN's quant as C converts it, undefined, where Rust's `as` gives 0:
+    no NaN there.)"""
+    def edit(h):
+        h[1] = 0.0
+        h[2] *= np.float32(1e30)
+        h[3] *= np.float32(1e-30)
+        h[4, 5] = np.inf
+        if types[0] == Q8_0:
+            h[5, 7] = np.nan
+    with np.errstate(all="ignore"):
+        run(orc, engine, types, 2048, 1536, (T,), edit)
