@@ -638,6 +638,12 @@ int forward(biv_hip_ctx *ctx, const biv_hip_moe *m, const float *h, int T, float
         ra.xh = reinterpret_cast<uint4 *>(s.xh);
         ra.xl = reinterpret_cast<uint4 *>(s.xl);
     }
+    // the exact gate/up on the matrix cores takes the Q8 of h as f16 (in the
+    // bf16 halves' buffer, which such a layer's gate/up does not use)
+    if (mq_gu) {
+        ra.f16 = 1;
+        ra.xq = reinterpret_cast<int8_t *>(s.xh);
+    }
     // BF16 gate/up (routed and shared) read h as f32 or as its bf16 halves:
     // nothing reads the Q8 of h, so the router launch leaves it out
     if (m->gate->m.ty == biv::T_BF16 && (!has_shared || m->sg->m.ty == biv::T_BF16)) ra.xq = nullptr;
@@ -714,6 +720,7 @@ int forward(biv_hip_ctx *ctx, const biv_hip_moe *m, const float *h, int T, float
             HIP_TRY(ctx, biv::launch_mfma_gateup(g, st), "expert gate/up (mfma)");
         } else if (mq_gu) {
             a.sh_chunk = biv::MFMA_Q8_TILE;
+            a.xq = ra.xq;
             HIP_TRY(ctx, biv::launch_mfma_gateup_exact(a, st), "expert gate/up (int8 mfma)");
         } else {
             HIP_TRY(ctx, biv::launch_gateup(a, st), "expert gate/up");

@@ -76,6 +76,7 @@ struct RouterArgs {
     float *glogit;         // [T]
     int8_t *xq;            // h quantised: [T][E] chain layout
     float *xd, *xs;        // [T][E/32]
+    int f16;               // h quantised as launch_quant_f16 writes it instead (xq: [T][E] f16)
     // With norm_w: h is the residual x and every use of it takes
     // rms_norm(x) (ops.rs:136-144) with these weights and eps, the
     // post_norm before the FFN (model.rs:786-790); hn [T][E] receives it.
@@ -213,8 +214,8 @@ hipError_t launch_mfma_down(const MfArgs &a, hipStream_t st);
 // Quantised experts at prefill sizes on the int8 matrix cores (mfma.hip),
 // with the chain kernels' contract (MvArgs: Q8 input rows a.xq / a.xd / a.xs,
 // f32 out, dump taps) and slots of at most MFMA_Q8_TILE pairs.  gate/up
-// (Q8_0 or Q4_K; gate and up of one type): bit for bit the x86 order, the
-// MFMAs making the 4-element word dots.  down (Q8_0 or Q6_K):
+// (exact.hip; Q8_0 or Q4_K, gate and up of one type; the Q8 rows in
+// launch_quant_f16's order): bit for bit the x86 order.  down (Q8_0 or Q6_K):
 // exact int32 block dots (Q6_K: 16-element halves times their sub-scales),
 // f32 sums over blocks in an order of their own.
 constexpr int MFMA_Q8_TILE = 16;

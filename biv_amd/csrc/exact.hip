@@ -412,6 +412,202 @@ __global__ __launch_bounds__(EX_NTH) __attribute__((amdgpu_waves_per_eu(ex_waves
     run(std::integral_constant<int, 1>());
 }
 
+// ---------------------------------------------------------------------------
+// The experts' gate/up at prefill sizes (Q8_0, Q4_K), the same sums over a
+// slot of up to 16 pairs.
+//
+// Here the weights are met by one slot only and come from HBM, so what counts
+// besides the chains' FMAs is that their loads run far ahead: a workgroup
+// stages its pairs' whole rows once (f16, 64 KB at K = 2048, by DMA), and
+// after that one barrier its waves run free, each streaming 16 rows of gate
+// and the same 16 of up with loads three of four steps ahead in registers (a
+// step: one matrix, one parity of 256 elements; Q4_K: both).  A wave holds
+// both matrices' chains of the 16 pairs (128 accumulators), so the tree and
+// the SwiGLU need no exchange between lanes.
+constexpr int GS_WAVES = 4;
+constexpr int GS_NTH = 64 * GS_WAVES;
+constexpr int GS_ROWS = MFMA_Q8_TILE;       // pairs of a slot
+constexpr int GS_ROWS_WG = 16 * GS_WAVES;   // output rows of a workgroup
+static_assert(GS_ROWS == 16, "one tile of pairs");
+
+template <int TY, int K, bool DUMP>
+__global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1 : 2))) void k_gu_slot(MvArgs a)
+{
+    using W = ExW<TY>;
+    constexpr bool Q4 = TY == T_Q4K;
+    constexpr int NB = K / 32, NG = K / EX_KC;
+    constexpr int X = GS_ROWS * 2 * K, S = NB * GS_ROWS * 4;
+    // a pair's row as 16-byte pieces, piece p of row r at p ^ r (low four
+    // bits): 16 lanes reading one piece of 16 rows fall in 64 banks; then the
+    // block scales (and Q4_K's block sums) [block][pair]
+    __shared__ __align__(16) uint8_t lds[X + S * (Q4 ? 2 : 1)];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lg = lane >> 4, lc = lane & 15;
+    int u, rt;
+    if (!slot_unit<SLOT_RUN>(a, blockIdx.x, u, rt)) return;
+    const bool shared = u < a.n_sh;
+    int e = 0, beg, cnt, tok0 = 0;
+    if (shared) {
+        tok0 = u * a.sh_chunk;
+        beg = a.P + tok0;
+        cnt = min(a.sh_chunk, a.T - tok0);
+    } else {
+        const Slot &sl = a.dp.slots[u - a.n_sh];
+        cnt = __builtin_amdgcn_readfirstlane(sl.cnt);
+        if (cnt == 0) return;
+        e = __builtin_amdgcn_readfirstlane(sl.expert);
+        beg = __builtin_amdgcn_readfirstlane(sl.beg);
+    }
+    const DevMat Mg = shared ? a.sa : a.a, Mu = shared ? a.sb : a.b;
+    const int rows = Mg.rows, orow = rt * GS_ROWS_WG + 16 * wave + lc;
+    const size_t wrow = (size_t)e * rows + orow;
+    // lane lc's pair (past the count the last one)
+    const int ti = min(lc, cnt - 1), tok = shared ? tok0 + ti : a.dp.pair_tok[beg + ti];
+    // the weights of steps: w[i][mat][pi] of 256-element group g + i (Q4_K:
+    // both parities in pi 0, two groups a turn)
+    constexpr int NP = Q4 ? 1 : 2, NU = Q4 ? 2 : 1;
+    W w[NU][2][NP];
+#pragma unroll
+    for (int i = 0; i < NU; i++)
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            w[i][0][p].load(Mg, wrow, K, i, lg, p);
+            w[i][1][p].load(Mu, wrow, K, i, lg, p);
+        }
+    {
+        const unsigned lds0 = lds_addr(lds);
+        const uint8_t *xh = reinterpret_cast<const uint8_t *>(a.xq);
+        // rows past the count stay as they are (their results are not stored)
+#pragma unroll
+        for (int q = 0; q < GS_ROWS / GS_WAVES; q++) {
+            const int r = GS_WAVES * q + wave;
+            if (r >= cnt) break; // uniform over the wave
+            const uint8_t *src = xh + (size_t)(uint32_t)__builtin_amdgcn_readlane(tok, r) * (2 * K);
+#pragma unroll
+            for (int i = 0; i < K / 512; i++)
+                lds_dma16_off(src, 16 * ((64 * i + lane) ^ r), lds0 + r * 2 * K + 1024 * i);
+        }
+        const size_t so = (size_t)tok * NB + lg; // four blocks of 16 pairs an instruction
+#pragma unroll
+        for (int q = 0; q < NB / 4 / GS_WAVES; q++) {
+            const int b4 = GS_WAVES * q + wave;
+            lds_dma4_at(a.xd + so + 4 * b4, lds0 + X + 256 * b4);
+            if (Q4) lds_dma4_at(a.xs + so + 4 * b4, lds0 + X + S + 256 * b4);
+        }
+    }
+    wait_vm<0>();
+    __syncthreads();
+    float acc[2][4][2][8], mins[2][4]; // [matrix][row][parity][word]
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            mins[m][r] = 0.0f;
+#pragma unroll
+            for (int l = 0; l < 8; l++) acc[m][r][0][l] = acc[m][r][1][l] = 0.0f;
+        }
+    const f32x16 z = {};
+    const float *dl = reinterpret_cast<const float *>(lds + X) + 16 * 2 * lg + lc;
+    const float *sl = reinterpret_cast<const float *>(lds + X + (Q4 ? S : 0)) + 16 * lg + lc;
+    auto step = [&](const W &wm, int g, auto m_c, auto pi_c) {
+        constexpr int m = decltype(m_c)::value, pi = decltype(pi_c)::value;
+        if constexpr (Q4) if constexpr (pi == 0) {
+            // mins += dmin * (m_a * s_a + m_b * s_b) over the sub-block pairs
+            // in order; four products m * s (rounded once, as written) in one
+            // k = 1 f32 MFMA
+            const float dm = wm.dmin();
+#pragma unroll
+            for (int hf = 0; hf < 2; hf++) {
+                const float mv = (float)((wm.six(1, hf) >> (8 * lg)) & 0xFF);
+                const f32x16 p = __builtin_amdgcn_mfma_f32_16x16x1f32(sl[16 * (8 * g + 4 * hf)], mv, z, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    mins[m][r] = mins[m][r] + dm * (p[r] + p[4 + r]);
+                    mins[m][r] = mins[m][r] + dm * (p[8 + r] + p[12 + r]);
+                }
+            }
+        }
+        // (the second matrix's step reads the activations again: kept from the
+        // first they take 16 registers)
+        int xo = lc * 2 * K;
+        asm volatile("" : "+v"(xo));
+        // w_scale * d_x of blocks 2 j + pi in registers 4 j + r
+        const f32x16 s = __builtin_amdgcn_mfma_f32_16x16x1f32(dl[16 * (8 * g + pi)], wm.wscale(lg, pi), z, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const f16x8 xa = *reinterpret_cast<const f16x8 *>(lds + xo + 16 * ((4 * (8 * g + 2 * j + pi) + lg) ^ lc));
+            int bdot[4] = {0, 0, 0, 0}; // (DUMP)
+#pragma unroll
+            for (int hh = 0; hh < 2; hh++) {
+                const f16x4 x4 = hh ? __builtin_shufflevector(xa, xa, 4, 5, 6, 7) : __builtin_shufflevector(xa, xa, 0, 1, 2, 3);
+                const f32x16 d = __builtin_amdgcn_mfma_f32_16x16x4f16(x4, wm.operand(j, hh, pi), z, 0, 0, 0);
+#pragma unroll
+                for (int l = 0; l < 4; l++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        acc[m][r][pi][4 * hh + l] = __builtin_fmaf(d[4 * l + r], s[4 * j + r], acc[m][r][pi][4 * hh + l]);
+                if (DUMP)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) bdot[r] += (int)d[r] + (int)d[4 + r] + (int)d[8 + r] + (int)d[12 + r];
+            }
+            int32_t *dump = DUMP ? (m ? a.dump_b : a.dump_a) : nullptr;
+            if (DUMP && dump) { // the block dots, for the taps
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (4 * lg + r < cnt)
+                        dump[((size_t)(beg + 4 * lg + r) * rows + orow) * NB + 8 * g + 2 * j + pi] = bdot[r];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0); // (steps one by one: registers)
+    };
+    const std::integral_constant<int, 0> c0;
+    const std::integral_constant<int, 1> c1;
+    // the group count as a value the compiler cannot see through (a.T is
+    // never negative): a loop of one or two turns it would lay out flat, the
+    // turns' loads and chains overlapped past the registers
+    const int ng = NG + (a.T < 0 ? 2 : 0);
+#pragma unroll 1
+    for (int g = 0; g < ng; g += NU)
+#pragma unroll
+        for (int i = 0; i < NU; i++) {
+            // (past the end the last group again, unused: no branch here)
+            const int gn = min(g + i + NU, NG - 1);
+            if constexpr (Q4) {
+                step(w[i][0][0], g + i, c0, c0);
+                step(w[i][0][0], g + i, c0, c1);
+                w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
+                step(w[i][1][0], g + i, c1, c0);
+                step(w[i][1][0], g + i, c1, c1);
+                w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
+            } else {
+                step(w[i][0][0], g + i, c0, c0);
+                w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
+                step(w[i][1][0], g + i, c1, c0);
+                w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
+                step(w[i][0][NP - 1], g + i, c0, c1);
+                w[i][0][NP - 1].load(Mg, wrow, K, gn, lg, 1);
+                step(w[i][1][NP - 1], g + i, c1, c1);
+                w[i][1][NP - 1].load(Mu, wrow, K, gn, lg, 1);
+            }
+        }
+    // the reference's tree (chains pi, then l 4, 2 and 1 apart), the mins,
+    // and silu(gate) * up
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        float y[2];
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            float v[4];
+#pragma unroll
+            for (int l = 0; l < 4; l++)
+                v[l] = (acc[m][r][0][l] + acc[m][r][1][l]) + (acc[m][r][0][l + 4] + acc[m][r][1][l + 4]);
+            y[m] = (v[0] + v[2]) + (v[1] + v[3]);
+            if (Q4) y[m] = y[m] - mins[m][r];
+        }
+        if (4 * lg + r < cnt) a.out[(size_t)(beg + 4 * lg + r) * rows + orow] = silu_mul_t(y[0], y[1], exp_tab);
+    }
+}
+
 } // namespace
 
 constexpr int N_CU = 256;
@@ -461,6 +657,47 @@ hipError_t launch_exact(const ExactArgs &a, int gateup, hipStream_t st)
     BIV_EX_CASE(T_Q6K)
 #undef BIV_EX_CASE
     return hipErrorInvalidValue;
+}
+
+static hipError_t launch_gu_t(MvArgs a, int routed, int shared, hipStream_t st)
+{
+    const DevMat &M = routed ? a.a : a.sa;
+    if (!routed) a.u_max = 0;
+    a.n_sh = shared ? (a.T + a.sh_chunk - 1) / a.sh_chunk : 0;
+    const int slots = a.u_max + a.n_sh;
+    if (slots == 0) return hipSuccess;
+    if (a.sh_chunk > GS_ROWS || M.rows % GS_ROWS_WG) return hipErrorInvalidValue;
+    a.n_rt = M.rows / GS_ROWS_WG;
+    const dim3 grid(slot_grid<SLOT_RUN>(slots, a.n_rt));
+    const bool dump = a.dump_a || a.dump_b;
+#define BIV_GU_CASE(TY, KK)                                                                                     \
+    if (M.ty == TY && M.cols == KK) {                                                                           \
+        if (dump)                                                                                               \
+            k_gu_slot<TY, KK, true><<<grid, GS_NTH, 0, st>>>(a);                                                 \
+        else                                                                                                    \
+            k_gu_slot<TY, KK, false><<<grid, GS_NTH, 0, st>>>(a);                                                \
+        return hipGetLastError();                                                                               \
+    }
+    BIV_GU_CASE(T_Q8_0, 2048)
+    BIV_GU_CASE(T_Q8_0, 1024)
+    BIV_GU_CASE(T_Q8_0, 512)
+    BIV_GU_CASE(T_Q4K, 2048)
+    BIV_GU_CASE(T_Q4K, 1024)
+    BIV_GU_CASE(T_Q4K, 512)
+#undef BIV_GU_CASE
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_mfma_gateup_exact(const MvArgs &a, hipStream_t st)
+{
+    // routed and shared in one launch when they share a type and shape
+    const bool has_shared = a.sa.q != nullptr;
+    if (a.a.ty != a.b.ty || (has_shared && a.sa.ty != a.sb.ty)) return hipErrorInvalidValue;
+    if (has_shared && a.sa.ty == a.a.ty && a.sa.cols == a.a.cols && a.sa.rows == a.a.rows)
+        return launch_gu_t(a, 1, 1, st);
+    hipError_t err = launch_gu_t(a, 1, 0, st);
+    if (err != hipSuccess || !has_shared) return err;
+    return launch_gu_t(a, 0, 1, st);
 }
 
 } // namespace biv

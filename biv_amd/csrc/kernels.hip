@@ -120,10 +120,25 @@ __device__ inline void quant_block_at(const float (&v)[32], int K, int b, int *q
     if (srow) srow[lay::q8_scale(K, b)] = s;
 }
 
-// The same from a block in LDS, read twice (amax, then the quants) so that
+// where the f16 order (launch_quant_f16) has word l of block b, in 8-byte units
+__device__ constexpr int f16_word(int b, int l) { return 8 * b + 2 * (l & 3) + (l >> 2); }
+// quant_block_at in that order
+__device__ inline void quant_block_f16(const float (&v)[32], int b, uint2 *qrow, float *drow, float *srow)
+{
+    unsigned q[8];
+    quant_words(v, q, drow[b], srow[b]);
+    uint4 *o = reinterpret_cast<uint4 *>(qrow + 8 * b);
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+        const uint2 x = i8x4_to_f16x4(q[l]), y = i8x4_to_f16x4(q[l + 4]);
+        o[l] = make_uint4(x.x, x.y, y.x, y.y);
+    }
+}
+
+// The same (f16: in that order) from a block in LDS, read twice (amax, then the quants) so that
 // few registers are live; 16-byte word l of the block at v[l ^ sw].
 __device__ inline void quant_block_lds(const float4 *v, int K, int b, int *qrow, float *drow, float *srow = nullptr,
-                                       int sw = 0)
+                                       int sw = 0, bool f16 = false)
 {
     float amax = 0.0f;
 #pragma unroll
@@ -148,14 +163,19 @@ __device__ inline void quant_block_lds(const float4 *v, int K, int b, int *qrow,
         sum += r3;
         const unsigned w = ((unsigned)r0 & 0xFF) | (((unsigned)r1 & 0xFF) << 8) | (((unsigned)r2 & 0xFF) << 16) |
                            (((unsigned)r3 & 0xFF) << 24);
-        qrow[lay::q8_word(b, l)] = (int)w;
+        if (f16) reinterpret_cast<uint2 *>(qrow)[f16_word(b, l)] = i8x4_to_f16x4(w);
+        else qrow[lay::q8_word(b, l)] = (int)w;
     }
-    drow[lay::q8_scale(K, b)] = db;
-    if (srow) srow[lay::q8_scale(K, b)] = db * (float)sum;
+    const int sb = f16 ? b : lay::q8_scale(K, b);
+    drow[sb] = db;
+    if (srow) srow[sb] = db * (float)sum;
 }
 
-__device__ inline void quant_block(const float (&v)[32], int K, size_t row, int b, int8_t *qs, float *d, float *s)
+__device__ inline void quant_block(const float (&v)[32], int K, size_t row, int b, int8_t *qs, float *d, float *s,
+                                   bool f16 = false)
 {
+    if (f16)
+        return quant_block_f16(v, b, reinterpret_cast<uint2 *>(qs + row * K * 2), d + row * (K / 32), s + row * (K / 32));
     quant_block_at(v, K, b, reinterpret_cast<int *>(qs + row * K), d + row * (K / 32), s + row * (K / 32));
 }
 
@@ -275,7 +295,7 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
                     v[4 * j + 3] = v[4 * j + 3] * (scale * w.w);
                     o4[j] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
                 }
-                if (a.xq) quant_block(v, E, t, b, a.xq, a.xd, a.xs);
+                if (a.xq) quant_block(v, E, t, b, a.xq, a.xd, a.xs, a.f16);
             }
         }
         return;
@@ -286,7 +306,7 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
              i += nthreads) {
             float v[32];
             load32(h + 32 * (size_t)i, v);
-            quant_block(v, E, i / (E / 32), i % (E / 32), a.xq, a.xd, a.xs);
+            quant_block(v, E, i / (E / 32), i % (E / 32), a.xq, a.xd, a.xs, a.f16);
         }
         return;
     }
@@ -822,8 +842,8 @@ template <int NS> __global__ __launch_bounds__(64 * PREP_TOK) void k_prep(Router
     wave_lds_sync();
     if (a.xq && lane < NS)
         quant_block_lds(reinterpret_cast<const float4 *>(r + lane * PREP_PITCH), E, lane,
-                        reinterpret_cast<int *>(a.xq + (size_t)t * E), a.xd + (size_t)t * (E / 32),
-                        a.xs + (size_t)t * (E / 32));
+                        reinterpret_cast<int *>(a.xq + (size_t)t * E * (a.f16 ? 2 : 1)), a.xd + (size_t)t * (E / 32),
+                        a.xs + (size_t)t * (E / 32), 0, a.f16);
     if (a.xh) {
         // the bf16 halves for the matrix-core gate/up: 16-byte chunk 16 g + c
         // of the row holds elements 128 g + 16 m + c, m = 0..7
@@ -2483,14 +2503,7 @@ __global__ __launch_bounds__(256) void k_quant_f16(const float *__restrict__ x, 
     if (i >= n_blocks) return;
     float v[32];
     load32(x + 32 * (size_t)i, v);
-    unsigned q[8];
-    quant_words(v, q, d[i], s[i]);
-    uint4 *o = reinterpret_cast<uint4 *>(xh + 32 * (size_t)i);
-#pragma unroll
-    for (int l = 0; l < 4; l++) {
-        const uint2 a = i8x4_to_f16x4(q[l]), b = i8x4_to_f16x4(q[l + 4]);
-        o[l] = make_uint4(a.x, a.y, b.x, b.y);
-    }
+    quant_block_f16(v, 0, reinterpret_cast<uint2 *>(xh + 32 * (size_t)i), d + i, s + i);
 }
 
 // The combine as its own launch: grid (E / 256, T).

@@ -27,18 +27,36 @@ __device__ inline void lds_dma16_at(const void *g, unsigned lds_addr)
     const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_addr);
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(m0) : "memory", "m0");
 }
+// The same, one dword per lane (LDS address m0 + 4 lane).
+__device__ inline void lds_dma4_at(const void *g, unsigned lds_addr)
+{
+    const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_addr);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(m0) : "memory", "m0");
+}
 // The same from a uniform base and a 32-bit byte offset per lane, 16 bytes or
 // one dword (LDS address m0 + 4 lane) a lane.
-__device__ inline void lds_dma16_off(const void *base, uint32_t off, unsigned lds_addr)
+__device__ inline uint64_t uniform_addr(const void *p)
 {
+    // (the compiler may keep a uniform pointer in vector registers; an SGPR
+    // that a vector instruction writes may be read as a load's base only five
+    // wait states later, which the compiler does not see to inside inline asm:
+    // the users' s_nop)
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)), lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    return (uint64_t)hi << 32 | lo; // (the builtin's int would sign-extend)
+}
+__device__ inline void lds_dma16_off(const void *p, uint32_t off, unsigned lds_addr)
+{
+    const uint64_t base = uniform_addr(p);
     const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_addr);
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0)
                  : "memory", "m0");
 }
-__device__ inline void lds_dma4_off(const void *base, uint32_t off, unsigned lds_addr)
+__device__ inline void lds_dma4_off(const void *p, uint32_t off, unsigned lds_addr)
 {
+    const uint64_t base = uniform_addr(p);
     const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_addr);
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0)
                  : "memory", "m0");
 }
 // the LDS address (byte offset) of a shared-memory pointer
