@@ -29,6 +29,8 @@
 // rows, so a weight word is converted to f16 once for 64 input rows (10
 // instructions per block and lane against 128 FMAs), and the activations are
 // written as f16 once by the quantiser and arrive in LDS by DMA.
+#include <type_traits>
+
 #include "common.hpp"
 #include "layout.hpp"
 #include "lds_dma.hpp"
@@ -48,28 +50,40 @@ __device__ __forceinline__ f16x4 as_f16x4(const uint2 &v) { return __builtin_bit
 // operand(j, hh) is word 4 hh + lg of block pi + 2 j as four exact f16;
 // wscale() the f32 scale of block pi + 2 lg as the reference forms it.  (pi
 // is uniform over the wave.)
-template <int TY> struct ExW;
+// ALL: the scales of the four blocks in every lane (scale(j, pi)).
+template <int TY, bool ALL = false> struct ExW;
 
 // Q8_0 (chain layout: unit 16 g + 8 pi + w holds word w of blocks 8 g + pi +
 // 2 j, j = 0..3); scale f16(d)
-template <> struct ExW<T_Q8_0> {
+template <bool ALL> struct ExW<T_Q8_0, ALL> {
     uint4 q[2];
-    uint16_t s;
+    std::conditional_t<ALL, uint2, uint16_t> s;
     __device__ __forceinline__ void load(const DevMat &M, size_t row, int K, int g, int lg, int pi)
     {
         const uint4 *p = reinterpret_cast<const uint4 *>(M.q + row * K) + 16 * g + 8 * pi + lg;
         q[0] = p[0];
         q[1] = p[4];
-        s = reinterpret_cast<const uint16_t *>(M.s + row * (K / 16))[pi * (K / 64) + 4 * g + lg];
+        const uint16_t *ps = reinterpret_cast<const uint16_t *>(M.s + row * (K / 16)) + pi * (K / 64) + 4 * g;
+        if constexpr (ALL) s = *reinterpret_cast<const uint2 *>(ps);
+        else s = ps[lg];
     }
     __device__ __forceinline__ f16x4 operand(int j, int hh, int) const { return as_f16x4(i8x4_to_f16x4(q[hh][j])); }
-    __device__ __forceinline__ float wscale(int, int) const { return f16_to_f32(s); }
+    __device__ __forceinline__ float wscale(int lg, int) const
+    {
+        if constexpr (ALL) return f16_to_f32((uint32_t)(((uint64_t)s.y << 32 | s.x) >> (16 * lg)) & 0xFFFF);
+        else return f16_to_f32(s);
+    }
+    __device__ __forceinline__ float scale(int j, int) const
+    {
+        const uint32_t h2 = j < 2 ? s.x : s.y;
+        return f16_to_f32((j & 1) ? h2 >> 16 : h2 & 0xFFFF);
+    }
 };
 
 // Q4_K (chain layout: unit 8 g + w holds word w of the four sub-block pairs
 // of super-block g, low nibbles the even sub-block, high the odd); scale d *
 // sc of the sub-block, the mins apart
-template <> struct ExW<T_Q4K> {
+template <bool ALL> struct ExW<T_Q4K, ALL> {
     uint4 q[2];
     uint4 hd; // d, dmin, the 12 scale bytes
     __device__ __forceinline__ void load(const DevMat &M, size_t row, int K, int g, int lg, int)
@@ -95,6 +109,10 @@ template <> struct ExW<T_Q4K> {
         const uint64_t sc = (uint64_t)six(0, 1) << 32 | six(0, 0);
         return f16_to_f32(hd.x & 0xFFFF) * (float)((uint32_t)(sc >> (8 * (2 * lg + pi))) & 0xFF);
     }
+    __device__ __forceinline__ float scale(int j, int pi) const
+    {
+        return f16_to_f32(hd.x & 0xFFFF) * (float)((six(0, j >> 1) >> (8 * (2 * (j & 1) + pi))) & 0xFF);
+    }
     __device__ __forceinline__ float dmin() const { return f16_to_f32(hd.x >> 16); }
 };
 
@@ -104,7 +122,7 @@ template <> struct ExW<T_Q4K> {
 // half j >> 1.  The word's sub-scale goes into the operand: (q - 32) * sc as
 // (q - 32) * 16 (sc >> 4) plus (q - 32) * (sc & 15), both exact in f16, in
 // two MFMAs whose sum is the exact integer.  Scale d.
-template <> struct ExW<T_Q6K> {
+template <bool ALL> struct ExW<T_Q6K, ALL> {
     uint2 ql[2], qh[2];
     uint32_t sc[2]; // [hh], a byte per step
     uint16_t d;
@@ -433,7 +451,7 @@ static_assert(GS_ROWS == 16, "one tile of pairs");
 template <int TY, int K, bool DUMP>
 __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1 : 2))) void k_gu_slot(MvArgs a)
 {
-    using W = ExW<TY>;
+    using W = ExW<TY, true>;
     constexpr bool Q4 = TY == T_Q4K;
     constexpr int NB = K / 32, NG = K / EX_KC;
     constexpr int X = GS_ROWS * 2 * K, S = NB * GS_ROWS * 4;
@@ -497,114 +515,284 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
     }
     wait_vm<0>();
     __syncthreads();
-    float acc[2][4][2][8], mins[2][4]; // [matrix][row][parity][word]
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            mins[m][r] = 0.0f;
-#pragma unroll
-            for (int l = 0; l < 8; l++) acc[m][r][0][l] = acc[m][r][1][l] = 0.0f;
-        }
     const f32x16 z = {};
-    const float *dl = reinterpret_cast<const float *>(lds + X) + 16 * 2 * lg + lc;
-    const float *sl = reinterpret_cast<const float *>(lds + X + (Q4 ? S : 0)) + 16 * lg + lc;
-    auto step = [&](const W &wm, int g, auto m_c, auto pi_c) {
-        constexpr int m = decltype(m_c)::value, pi = decltype(pi_c)::value;
-        if constexpr (Q4) if constexpr (pi == 0) {
-            // mins += dmin * (m_a * s_a + m_b * s_b) over the sub-block pairs
-            // in order; four products m * s (rounded once, as written) in one
-            // k = 1 f32 MFMA
-            const float dm = wm.dmin();
+    const f32x4 z4 = {};
+    const std::integral_constant<int, 0> c0;
+    const std::integral_constant<int, 1> c1;
+    auto at = [&](int o) { return reinterpret_cast<const float *>(lds + o); };
+    // The steps of every group in turn, each followed by the load of the same
+    // step of a later group (past the end the last one again, unused: no
+    // branch in the loop); step(weights, matrix, parity) is followed by
+    // advance() once a group.
+    auto walk = [&](auto step, auto advance) {
+        // the group count as a value the compiler cannot see through (a.T is
+        // never negative): a loop of one or two turns it would lay out flat,
+        // the turns' loads and chains overlapped past the registers
+        const int ng = NG + (a.T < 0 ? 2 : 0);
+#pragma unroll 1
+        for (int g = 0; g < ng; g += NU)
 #pragma unroll
-            for (int hf = 0; hf < 2; hf++) {
-                const float mv = (float)((wm.six(1, hf) >> (8 * lg)) & 0xFF);
-                const f32x16 p = __builtin_amdgcn_mfma_f32_16x16x1f32(sl[16 * (8 * g + 4 * hf)], mv, z, 0, 0, 0);
+            for (int i = 0; i < NU; i++) {
+                const int gn = min(g + i + NU, NG - 1);
+                if constexpr (Q4) {
+                    step(w[i][0][0], g + i, c0, c0);
+                    step(w[i][0][0], g + i, c0, c1);
+                    w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
+                    step(w[i][1][0], g + i, c1, c0);
+                    step(w[i][1][0], g + i, c1, c1);
+                    w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
+                } else {
+                    step(w[i][0][0], g + i, c0, c0);
+                    w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
+                    step(w[i][1][0], g + i, c1, c0);
+                    w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
+                    step(w[i][0][NP - 1], g + i, c0, c1);
+                    w[i][0][NP - 1].load(Mg, wrow, K, gn, lg, 1);
+                    step(w[i][1][NP - 1], g + i, c1, c1);
+                    w[i][1][NP - 1].load(Mu, wrow, K, gn, lg, 1);
+                }
+                advance();
+            }
+    };
+    auto dump = [&](int m, int row, int b, int v) { // the block dots, for the taps
+        int32_t *d = m ? a.dump_b : a.dump_a;
+        if (d && row < cnt) d[((size_t)(beg + row) * rows + orow) * NB + b] = v;
+    };
+    // Slots of more than 8 pairs: 16-row tiles.
+    auto run16 = [&]() {
+        float acc[2][4][2][8], mins[2][4]; // [matrix][row][parity][word]
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    mins[m][r] = mins[m][r] + dm * (p[r] + p[4 + r]);
-                    mins[m][r] = mins[m][r] + dm * (p[8 + r] + p[12 + r]);
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                mins[m][r] = 0.0f;
+#pragma unroll
+                for (int l = 0; l < 8; l++) acc[m][r][0][l] = acc[m][r][1][l] = 0.0f;
+            }
+        // byte offsets in LDS, 512 a group: the lane's pieces of blocks 2 j +
+        // pi (j & 1; j >> 1 is 256 bytes on), its block scale and block sum
+        int xo[2][2], dlo = X + 128 * lg + 4 * lc, slo = X + S + 64 * lg + 4 * lc;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int p = 0; p < 2; p++) xo[j][p] = lc * 2 * K + 16 * ((8 * j + 4 * p + lg) ^ lc);
+        auto step = [&](const W &wm, int g, auto m_c, auto pi_c) {
+            constexpr int m = decltype(m_c)::value, pi = decltype(pi_c)::value;
+            if constexpr (Q4) if constexpr (pi == 0) {
+                // mins += dmin * (m_a * s_a + m_b * s_b) over the sub-block
+                // pairs in order; four products m * s (rounded once, as
+                // written) in one k = 1 f32 MFMA
+                const float dm = wm.dmin();
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++) {
+                    const float mv = (float)((wm.six(1, hf) >> (8 * lg)) & 0xFF);
+                    const f32x16 p = __builtin_amdgcn_mfma_f32_16x16x1f32(*at(slo + 256 * hf), mv, z, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        mins[m][r] = mins[m][r] + dm * (p[r] + p[4 + r]);
+                        mins[m][r] = mins[m][r] + dm * (p[8 + r] + p[12 + r]);
+                    }
                 }
             }
-        }
-        // (the second matrix's step reads the activations again: kept from the
-        // first they take 16 registers)
-        int xo = lc * 2 * K;
-        asm volatile("" : "+v"(xo));
-        // w_scale * d_x of blocks 2 j + pi in registers 4 j + r
-        const f32x16 s = __builtin_amdgcn_mfma_f32_16x16x1f32(dl[16 * (8 * g + pi)], wm.wscale(lg, pi), z, 0, 0, 0);
+            // w_scale * d_x of blocks 2 j + pi in registers 4 j + r
+            const f32x16 s = __builtin_amdgcn_mfma_f32_16x16x1f32(*at(dlo + 64 * pi), wm.wscale(lg, pi), z, 0, 0, 0);
+            // (the second matrix's step reads the activations again: kept
+            // from the first they take 16 registers)
+            asm volatile("" : "+v"(xo[0][pi]), "+v"(xo[1][pi]));
+            // Unit u = 2 j + hh.  Q8_0: a unit's MFMA is issued before the
+            // FMAs of the one before it, which cover its latency (kernel at 512
+            // tokens 231 -> 219 us; Q4_K, whose mins and headers take the
+            // registers that needs, spills: 720 -> 888 at 2048).  LDS reads,
+            // weight loads and scalar work may cross the scheduling barriers.
+            constexpr bool AHEAD = !Q4;
+            constexpr int LOADS = 0x124; // SALU, VMEM reads, LDS reads
+            f16x8 xa[AHEAD ? 4 : 1];
+            auto read = [&](int j) { return *reinterpret_cast<const f16x8 *>(lds + xo[j & 1][pi] + 256 * (j >> 1)); };
+            if (AHEAD)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const f16x8 xa = *reinterpret_cast<const f16x8 *>(lds + xo + 16 * ((4 * (8 * g + 2 * j + pi) + lg) ^ lc));
+                for (int j = 0; j < 4; j++) xa[AHEAD ? j : 0] = read(j);
+            auto dots = [&](int u) {
+                const f16x8 v = xa[AHEAD ? u >> 1 : 0];
+                const f16x4 x4 = u & 1 ? __builtin_shufflevector(v, v, 4, 5, 6, 7) : __builtin_shufflevector(v, v, 0, 1, 2, 3);
+                return __builtin_amdgcn_mfma_f32_16x16x4f16(x4, wm.operand(u >> 1, u & 1, pi), z, 0, 0, 0);
+            };
+            f32x16 dn;
+            if (AHEAD) dn = dots(0);
             int bdot[4] = {0, 0, 0, 0}; // (DUMP)
 #pragma unroll
-            for (int hh = 0; hh < 2; hh++) {
-                const f16x4 x4 = hh ? __builtin_shufflevector(xa, xa, 4, 5, 6, 7) : __builtin_shufflevector(xa, xa, 0, 1, 2, 3);
-                const f32x16 d = __builtin_amdgcn_mfma_f32_16x16x4f16(x4, wm.operand(j, hh, pi), z, 0, 0, 0);
+            for (int u = 0; u < 8; u++) {
+                if (!AHEAD && !(u & 1)) xa[0] = read(u >> 1);
+                const f32x16 d = AHEAD ? dn : dots(u);
+                if (AHEAD && u < 7) dn = dots(u + 1);
+                if (AHEAD) __builtin_amdgcn_sched_barrier(LOADS);
 #pragma unroll
                 for (int l = 0; l < 4; l++)
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        acc[m][r][pi][4 * hh + l] = __builtin_fmaf(d[4 * l + r], s[4 * j + r], acc[m][r][pi][4 * hh + l]);
+                        acc[m][r][pi][4 * (u & 1) + l] =
+                            __builtin_fmaf(d[4 * l + r], s[4 * (u >> 1) + r], acc[m][r][pi][4 * (u & 1) + l]);
                 if (DUMP)
 #pragma unroll
-                    for (int r = 0; r < 4; r++) bdot[r] += (int)d[r] + (int)d[4 + r] + (int)d[8 + r] + (int)d[12 + r];
+                    for (int r = 0; r < 4; r++) {
+                        bdot[r] = (u & 1 ? bdot[r] : 0) + (int)d[r] + (int)d[4 + r] + (int)d[8 + r] + (int)d[12 + r];
+                        if (u & 1) dump(m, 4 * lg + r, 8 * g + 2 * (u >> 1) + pi, bdot[r]);
+                    }
+                if (AHEAD) __builtin_amdgcn_sched_barrier(LOADS);
             }
-            int32_t *dump = DUMP ? (m ? a.dump_b : a.dump_a) : nullptr;
-            if (DUMP && dump) { // the block dots, for the taps
+            __builtin_amdgcn_sched_barrier(0); // (steps one by one: registers)
+        };
+        walk(step, [&]() {
+            xo[0][0] += 512;
+            xo[0][1] += 512;
+            xo[1][0] += 512;
+            xo[1][1] += 512;
+            dlo += 512;
+            slo += 512;
+        });
+        // the reference's tree (chains pi, then l 4, 2 and 1 apart), the
+        // mins, and silu(gate) * up
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-                    if (4 * lg + r < cnt)
-                        dump[((size_t)(beg + 4 * lg + r) * rows + orow) * NB + 8 * g + 2 * j + pi] = bdot[r];
+        for (int r = 0; r < 4; r++) {
+            float y[2];
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                float v[4];
+#pragma unroll
+                for (int l = 0; l < 4; l++)
+                    v[l] = (acc[m][r][0][l] + acc[m][r][1][l]) + (acc[m][r][0][l + 4] + acc[m][r][1][l + 4]);
+                y[m] = (v[0] + v[2]) + (v[1] + v[3]);
+                if (Q4) y[m] = y[m] - mins[m][r];
             }
+            if (4 * lg + r < cnt) a.out[(size_t)(beg + 4 * lg + r) * rows + orow] = silu_mul_t(y[0], y[1], exp_tab);
         }
-        __builtin_amdgcn_sched_barrier(0); // (steps one by one: registers)
     };
-    const std::integral_constant<int, 0> c0;
-    const std::integral_constant<int, 1> c1;
-    // the group count as a value the compiler cannot see through (a.T is
-    // never negative): a loop of one or two turns it would lay out flat, the
-    // turns' loads and chains overlapped past the registers
-    const int ng = NG + (a.T < 0 ? 2 : 0);
-#pragma unroll 1
-    for (int g = 0; g < ng; g += NU)
+    // Slots of up to 8 pairs, in NQ groups of 4 rows (v_mfma_f32_4x4x4_16b_f16,
+    // whose 16 blocks are the words lg of 16 weight rows): lane (lg, lc) gets
+    // word lg of a group's row r and weight row lc in register r, so it holds
+    // the chains of words lg and 4 + lg, and the tree over lg runs across
+    // lanes 16 and 32 apart.
+    auto run4 = [&](auto nq_c) {
+        constexpr int NQ = decltype(nq_c)::value;
+        float acc[2][NQ][2][2][4], mins[2][NQ][4]; // [matrix][group][parity][half][row]
 #pragma unroll
-        for (int i = 0; i < NU; i++) {
-            // (past the end the last group again, unused: no branch here)
-            const int gn = min(g + i + NU, NG - 1);
-            if constexpr (Q4) {
-                step(w[i][0][0], g + i, c0, c0);
-                step(w[i][0][0], g + i, c0, c1);
-                w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
-                step(w[i][1][0], g + i, c1, c0);
-                step(w[i][1][0], g + i, c1, c1);
-                w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
-            } else {
-                step(w[i][0][0], g + i, c0, c0);
-                w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
-                step(w[i][1][0], g + i, c1, c0);
-                w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
-                step(w[i][0][NP - 1], g + i, c0, c1);
-                w[i][0][NP - 1].load(Mg, wrow, K, gn, lg, 1);
-                step(w[i][1][NP - 1], g + i, c1, c1);
-                w[i][1][NP - 1].load(Mu, wrow, K, gn, lg, 1);
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int q = 0; q < NQ; q++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    mins[m][q][r] = 0.0f;
+#pragma unroll
+                    for (int h = 0; h < 2; h++) acc[m][q][0][h][r] = acc[m][q][1][h][r] = 0.0f;
+                }
+        const int row = lane & 3; // the lane's row of each group, as an operand
+        int xo[NQ][2][2], dlo = X + 4 * row;
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+                    xo[q][j][p] = (4 * q + row) * 2 * K + 16 * ((8 * j + 4 * p + lg) ^ (4 * q + row));
+        auto step = [&](const W &wm, int g, auto m_c, auto pi_c) {
+            constexpr int m = decltype(m_c)::value, pi = decltype(pi_c)::value;
+            if constexpr (Q4) if constexpr (pi == 0) {
+                const float dm = wm.dmin();
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    float mv[2];
+#pragma unroll
+                    for (int o = 0; o < 2; o++) mv[o] = (float)((wm.six(1, j >> 1) >> (8 * (2 * (j & 1) + o))) & 0xFF);
+#pragma unroll
+                    for (int q = 0; q < NQ; q++) {
+                        f32x4 p[2];
+#pragma unroll
+                        for (int o = 0; o < 2; o++)
+                            p[o] = __builtin_amdgcn_mfma_f32_4x4x1f32(*at(dlo + S + 64 * (2 * j + o) + 16 * q), mv[o], z4, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) mins[m][q][r] = mins[m][q][r] + dm * (p[0][r] + p[1][r]);
+                    }
+                }
             }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float dw = wm.scale(j, pi);
+                f32x4 s[NQ];
+                f16x8 xa[NQ];
+                int bdot[NQ][4] = {}; // (DUMP)
+#pragma unroll
+                for (int q = 0; q < NQ; q++) {
+                    s[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(*at(dlo + 64 * (2 * j + pi) + 16 * q), dw, z4, 0, 0, 0);
+                    xa[q] = *reinterpret_cast<const f16x8 *>(lds + xo[q][j & 1][pi] + 256 * (j >> 1));
+                }
+#pragma unroll
+                for (int hh = 0; hh < 2; hh++) {
+                    const f16x4 b = wm.operand(j, hh, pi);
+#pragma unroll
+                    for (int q = 0; q < NQ; q++) {
+                        const f16x4 x4 = hh ? __builtin_shufflevector(xa[q], xa[q], 4, 5, 6, 7)
+                                            : __builtin_shufflevector(xa[q], xa[q], 0, 1, 2, 3);
+                        const f32x4 d = __builtin_amdgcn_mfma_f32_4x4x4f16(x4, b, z4, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            acc[m][q][pi][hh][r] = __builtin_fmaf(d[r], s[q][r], acc[m][q][pi][hh][r]);
+                            if (DUMP) bdot[q][r] += (int)d[r];
+                        }
+                    }
+                }
+                if (DUMP)
+#pragma unroll
+                    for (int q = 0; q < NQ; q++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            int v = bdot[q][r]; // of the lane's words: the four lanes' sum
+                            v += __shfl_xor(v, 16);
+                            v += __shfl_xor(v, 32);
+                            if (lg == 0) dump(m, 4 * q + r, 8 * g + 2 * j + pi, v);
+                        }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        walk(step, [&]() {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                xo[q][0][0] += 512;
+                xo[q][0][1] += 512;
+                xo[q][1][0] += 512;
+                xo[q][1][1] += 512;
+            }
+            dlo += 512;
+        });
+        // the tree, in every lane; lane lg then finishes row lg of each group
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            float y[2];
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                float t[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float v = (acc[m][q][0][0][r] + acc[m][q][1][0][r]) + (acc[m][q][0][1][r] + acc[m][q][1][1][r]);
+                    v = v + __shfl_xor(v, 32); // v0 + v2, v1 + v3
+                    t[r] = v + __shfl_xor(v, 16);
+                    if (Q4) t[r] = t[r] - mins[m][q][r];
+                }
+                y[m] = lg == 0 ? t[0] : lg == 1 ? t[1] : lg == 2 ? t[2] : t[3];
+            }
+            if (4 * q + lg < cnt) a.out[(size_t)(beg + 4 * q + lg) * rows + orow] = silu_mul_t(y[0], y[1], exp_tab);
         }
-    // the reference's tree (chains pi, then l 4, 2 and 1 apart), the mins,
-    // and silu(gate) * up
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        float y[2];
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            float v[4];
-#pragma unroll
-            for (int l = 0; l < 4; l++)
-                v[l] = (acc[m][r][0][l] + acc[m][r][1][l]) + (acc[m][r][0][l + 4] + acc[m][r][1][l + 4]);
-            y[m] = (v[0] + v[2]) + (v[1] + v[3]);
-            if (Q4) y[m] = y[m] - mins[m][r];
-        }
-        if (4 * lg + r < cnt) a.out[(size_t)(beg + 4 * lg + r) * rows + orow] = silu_mul_t(y[0], y[1], exp_tab);
+    };
+    // (uniform over the workgroup.  Everything is in already: the waits here
+    // tell the compiler so, whose merged view of the paths would otherwise
+    // make each turn of a loop wait for every load in flight.)
+    if (cnt > 8) {
+        wait_vm<0>();
+        run16();
+    } else if (cnt > 4) {
+        wait_vm<0>();
+        run4(std::integral_constant<int, 2>());
+    } else {
+        wait_vm<0>();
+        run4(std::integral_constant<int, 1>());
     }
 }
 
