@@ -459,6 +459,7 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
     // bits): 16 lanes reading one piece of 16 rows fall in 64 banks; then the
     // block scales (and Q4_K's block sums) [block][pair]
     __shared__ __align__(16) uint8_t lds[X + S * (Q4 ? 2 : 1)];
+    __shared__ uint64_t tab[32]; // expf's table, for the SwiGLU
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lg = lane >> 4, lc = lane & 15;
     int u, rt;
@@ -476,6 +477,7 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
         e = __builtin_amdgcn_readfirstlane(sl.expert);
         beg = __builtin_amdgcn_readfirstlane(sl.beg);
     }
+    if (tid < 32) tab[tid] = exp_tab[tid];
     const DevMat Mg = shared ? a.sa : a.a, Mu = shared ? a.sb : a.b;
     const int rows = Mg.rows, orow = rt * GS_ROWS_WG + 16 * wave + lc;
     const size_t wrow = (size_t)e * rows + orow;
@@ -651,6 +653,7 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
         });
         // the reference's tree (chains pi, then l 4, 2 and 1 apart), the
         // mins, and silu(gate) * up
+        float o[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             float y[2];
@@ -663,8 +666,11 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
                 y[m] = (v[0] + v[2]) + (v[1] + v[3]);
                 if (Q4) y[m] = y[m] - mins[m][r];
             }
-            if (4 * lg + r < cnt) a.out[(size_t)(beg + 4 * lg + r) * rows + orow] = silu_mul_t(y[0], y[1], exp_tab);
+            o[r] = silu_mul_t(y[0], y[1], tab);
         }
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (4 * lg + r < cnt) a.out[(size_t)(beg + 4 * lg + r) * rows + orow] = o[r];
     };
     // Slots of up to 8 pairs, in NQ groups of 4 rows (v_mfma_f32_4x4x4_16b_f16,
     // whose 16 blocks are the words lg of 16 weight rows): lane (lg, lc) gets
@@ -778,7 +784,8 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
                 }
                 y[m] = lg == 0 ? t[0] : lg == 1 ? t[1] : lg == 2 ? t[2] : t[3];
             }
-            if (4 * q + lg < cnt) a.out[(size_t)(beg + 4 * q + lg) * rows + orow] = silu_mul_t(y[0], y[1], exp_tab);
+            const float o = silu_mul_t(y[0], y[1], tab);
+            if (4 * q + lg < cnt) a.out[(size_t)(beg + 4 * q + lg) * rows + orow] = o;
         }
     };
     // (uniform over the workgroup.  Everything is in already: the waits here
