@@ -438,8 +438,9 @@ __global__ __launch_bounds__(EX_NTH) __attribute__((amdgpu_waves_per_eu(ex_waves
 // besides the chains' FMAs is that their loads run far ahead: a workgroup
 // stages its pairs' whole rows once (f16, 64 KB at K = 2048, by DMA), and
 // after that one barrier its waves run free, each streaming 16 rows of gate
-// and the same 16 of up with loads three of four steps ahead in registers (a
-// step: one matrix, one parity of 256 elements; Q4_K: both).  A wave holds
+// and the same 16 of up with the next group's loads in flight in registers
+// (three of four steps ahead, a step being one matrix and one parity of 256
+// elements; Q4_K, whose bytes hold both parities, two of four).  A wave holds
 // both matrices' chains of the 16 pairs (128 accumulators), so the tree and
 // the SwiGLU need no exchange between lanes.
 constexpr int GS_WAVES = 4;
@@ -483,17 +484,17 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
     const size_t wrow = (size_t)e * rows + orow;
     // lane lc's pair (past the count the last one)
     const int ti = min(lc, cnt - 1), tok = shared ? tok0 + ti : a.dp.pair_tok[beg + ti];
-    // the weights of steps: w[i][mat][pi] of 256-element group g + i (Q4_K:
-    // both parities in pi 0, two groups a turn)
-    constexpr int NP = Q4 ? 1 : 2, NU = Q4 ? 2 : 1;
-    W w[NU][2][NP];
+    // the weights of steps: w[mat][pi] of a 256-element group (Q4_K: both
+    // parities in pi 0).  (Two groups a turn for Q4_K, loads three steps
+    // ahead, double the loop's code, which narrow rows run through once:
+    // 512-wide layers 41 against 38 us.)
+    constexpr int NP = Q4 ? 1 : 2;
+    W w[2][NP];
 #pragma unroll
-    for (int i = 0; i < NU; i++)
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-            w[i][0][p].load(Mg, wrow, K, i, lg, p);
-            w[i][1][p].load(Mu, wrow, K, i, lg, p);
-        }
+    for (int p = 0; p < NP; p++) {
+        w[0][p].load(Mg, wrow, K, 0, lg, p);
+        w[1][p].load(Mu, wrow, K, 0, lg, p);
+    }
     {
         const unsigned lds0 = lds_addr(lds);
         const uint8_t *xh = reinterpret_cast<const uint8_t *>(a.xq);
@@ -522,39 +523,31 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
     const std::integral_constant<int, 0> c0;
     const std::integral_constant<int, 1> c1;
     auto at = [&](int o) { return reinterpret_cast<const float *>(lds + o); };
-    // The steps of every group in turn, each followed by the load of the same
-    // step of a later group (past the end the last one again, unused: no
-    // branch in the loop); step(weights, matrix, parity) is followed by
-    // advance() once a group.
+    // The steps of every group in turn, each matrix's (and for Q8_0 parity's)
+    // followed by the load of the same of the next group (past the end the
+    // last one again, unused: no branch in the loop); advance() ends a group.
     auto walk = [&](auto step, auto advance) {
         // the group count as a value the compiler cannot see through (a.T is
         // never negative): a loop of one or two turns it would lay out flat,
         // the turns' loads and chains overlapped past the registers
         const int ng = NG + (a.T < 0 ? 2 : 0);
 #pragma unroll 1
-        for (int g = 0; g < ng; g += NU)
-#pragma unroll
-            for (int i = 0; i < NU; i++) {
-                const int gn = min(g + i + NU, NG - 1);
-                if constexpr (Q4) {
-                    step(w[i][0][0], g + i, c0, c0);
-                    step(w[i][0][0], g + i, c0, c1);
-                    w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
-                    step(w[i][1][0], g + i, c1, c0);
-                    step(w[i][1][0], g + i, c1, c1);
-                    w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
-                } else {
-                    step(w[i][0][0], g + i, c0, c0);
-                    w[i][0][0].load(Mg, wrow, K, gn, lg, 0);
-                    step(w[i][1][0], g + i, c1, c0);
-                    w[i][1][0].load(Mu, wrow, K, gn, lg, 0);
-                    step(w[i][0][NP - 1], g + i, c0, c1);
-                    w[i][0][NP - 1].load(Mg, wrow, K, gn, lg, 1);
-                    step(w[i][1][NP - 1], g + i, c1, c1);
-                    w[i][1][NP - 1].load(Mu, wrow, K, gn, lg, 1);
-                }
-                advance();
+        for (int g = 0; g < ng; g++) {
+            const int gn = min(g + 1, NG - 1);
+            step(w[0][0], g, c0, c0);
+            if constexpr (Q4) step(w[0][0], g, c0, c1);
+            w[0][0].load(Mg, wrow, K, gn, lg, 0);
+            step(w[1][0], g, c1, c0);
+            if constexpr (Q4) step(w[1][0], g, c1, c1);
+            w[1][0].load(Mu, wrow, K, gn, lg, 0);
+            if constexpr (!Q4) {
+                step(w[0][NP - 1], g, c0, c1);
+                w[0][NP - 1].load(Mg, wrow, K, gn, lg, 1);
+                step(w[1][NP - 1], g, c1, c1);
+                w[1][NP - 1].load(Mu, wrow, K, gn, lg, 1);
             }
+            advance();
+        }
     };
     auto dump = [&](int m, int row, int b, int v) { // the block dots, for the taps
         int32_t *d = m ? a.dump_b : a.dump_a;
@@ -601,32 +594,26 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
             // (the second matrix's step reads the activations again: kept
             // from the first they take 16 registers)
             asm volatile("" : "+v"(xo[0][pi]), "+v"(xo[1][pi]));
-            // Unit u = 2 j + hh.  Q8_0: a unit's MFMA is issued before the
-            // FMAs of the one before it, which cover its latency (kernel at 512
-            // tokens 231 -> 219 us; Q4_K, whose mins and headers take the
-            // registers that needs, spills: 720 -> 888 at 2048).  LDS reads,
+            // Unit u = 2 j + hh: its MFMA is issued before the FMAs of the
+            // unit before it, which cover its latency (kernel alone: Q8_0 at
+            // 512 tokens 231 -> 219 us, Q4_K at 2048 644 -> 615).  LDS reads,
             // weight loads and scalar work may cross the scheduling barriers.
-            constexpr bool AHEAD = !Q4;
             constexpr int LOADS = 0x124; // SALU, VMEM reads, LDS reads
-            f16x8 xa[AHEAD ? 4 : 1];
-            auto read = [&](int j) { return *reinterpret_cast<const f16x8 *>(lds + xo[j & 1][pi] + 256 * (j >> 1)); };
-            if (AHEAD)
+            f16x8 xa[4];
 #pragma unroll
-                for (int j = 0; j < 4; j++) xa[AHEAD ? j : 0] = read(j);
+            for (int j = 0; j < 4; j++) xa[j] = *reinterpret_cast<const f16x8 *>(lds + xo[j & 1][pi] + 256 * (j >> 1));
             auto dots = [&](int u) {
-                const f16x8 v = xa[AHEAD ? u >> 1 : 0];
+                const f16x8 v = xa[u >> 1];
                 const f16x4 x4 = u & 1 ? __builtin_shufflevector(v, v, 4, 5, 6, 7) : __builtin_shufflevector(v, v, 0, 1, 2, 3);
                 return __builtin_amdgcn_mfma_f32_16x16x4f16(x4, wm.operand(u >> 1, u & 1, pi), z, 0, 0, 0);
             };
-            f32x16 dn;
-            if (AHEAD) dn = dots(0);
+            f32x16 dn = dots(0);
             int bdot[4] = {0, 0, 0, 0}; // (DUMP)
 #pragma unroll
             for (int u = 0; u < 8; u++) {
-                if (!AHEAD && !(u & 1)) xa[0] = read(u >> 1);
-                const f32x16 d = AHEAD ? dn : dots(u);
-                if (AHEAD && u < 7) dn = dots(u + 1);
-                if (AHEAD) __builtin_amdgcn_sched_barrier(LOADS);
+                const f32x16 d = dn;
+                if (u < 7) dn = dots(u + 1);
+                __builtin_amdgcn_sched_barrier(LOADS);
 #pragma unroll
                 for (int l = 0; l < 4; l++)
 #pragma unroll
@@ -639,7 +626,7 @@ __global__ __launch_bounds__(GS_NTH) __attribute__((amdgpu_waves_per_eu(DUMP ? 1
                         bdot[r] = (u & 1 ? bdot[r] : 0) + (int)d[r] + (int)d[4 + r] + (int)d[8 + r] + (int)d[12 + r];
                         if (u & 1) dump(m, 4 * lg + r, 8 * g + 2 * (u >> 1) + pi, bdot[r]);
                     }
-                if (AHEAD) __builtin_amdgcn_sched_barrier(LOADS);
+                __builtin_amdgcn_sched_barrier(LOADS);
             }
             __builtin_amdgcn_sched_barrier(0); // (steps one by one: registers)
         };
