@@ -253,8 +253,52 @@ __device__ inline float rms_scale(float acc, int n, float eps)
     return 1.0f / sqrtf(ss + eps);
 }
 
+// tokens up to which the router launch's post_norm and quantisation take a
+// wave per 16 blocks (past it there are waves enough with a half wave a token)
+constexpr int ROUTER_FEW_T = 16;
+
+// lane x's value from the lane next to it (x ^ 1), or two on (x ^ 2), of its four
+__device__ inline float quad_xor1(float x) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, true)); }
+__device__ inline float quad_xor2(float x) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, true)); }
+
+// quant_block of block b of token t by 4 adjacent lanes, lane `sub` of them
+// holding its elements 8 sub .. 8 sub + 7 (the largest magnitude and the
+// integer sum are exact in any order)
+__device__ inline void quant_quad(const float (&v)[8], int E, int t, int b, int sub, const RouterArgs &a)
+{
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) m = fmaxf(m, fabsf(v[j]));
+    m = fmaxf(m, quad_xor1(m));
+    m = fmaxf(m, quad_xor2(m));
+    const float db = m / 127.0f;
+    const float id = db != 0.0f ? 1.0f / db : 0.0f;
+    int sum = 0;
+    unsigned w[2] = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int r = (int)roundf(v[j] * id);
+        sum += r;
+        w[j >> 2] |= (unsigned)(r & 0xFF) << (8 * (j & 3));
+    }
+    sum += __builtin_amdgcn_mov_dpp(sum, 0xB1, 0xF, 0xF, true);
+    sum += __builtin_amdgcn_mov_dpp(sum, 0x4E, 0xF, 0xF, true);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if (a.f16) reinterpret_cast<uint2 *>(a.xq + (size_t)t * E * 2)[f16_word(b, 2 * sub + j)] = i8x4_to_f16x4(w[j]);
+        else reinterpret_cast<int *>(a.xq + (size_t)t * E)[lay::q8_word(b, 2 * sub + j)] = (int)w[j];
+    }
+    if (sub == 0) {
+        const size_t o = (size_t)t * (E / 32) + (a.f16 ? b : lay::q8_scale(E, b));
+        a.xd[o] = db;
+        a.xs[o] = db * (float)sum;
+    }
+}
+
 template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void k_router(RouterArgs a)
 {
+    // one token a workgroup (the 64-thread instances serve one token only)
+    constexpr bool ONE = TC == 1 || NTH == 64;
     constexpr int RPW = NTH / 32; // rows per workgroup (a half wave each)
     constexpr int E = 32 * NS;
     const float *__restrict__ router = a.router;
@@ -271,6 +315,37 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
         // per lane, and writes it to hn
         const int L = threadIdx.x & 31, nhw = NTH / 32;
         const int nq = gridDim.x - n_rw;
+        if (T <= ROUTER_FEW_T) {
+            // Few tokens: a wave per 16 blocks of a token, 4 lanes to a block
+            // (8 elements each), every load issued before the chain; each of
+            // a token's waves forms the scale for itself.  (A half wave per
+            // token, two whole blocks a lane one after the other, was the
+            // launch's longest path: T = 1 7.1 us against 3.2 without norm.)
+            constexpr int PARTS = NS / 16;
+            const int lane = threadIdx.x & 63, nw = NTH / 64;
+            for (int i = ((blockIdx.x - n_rw) * gridDim.y + blockIdx.y) * nw + (threadIdx.x >> 6); i < T * PARTS;
+                 i += nq * gridDim.y * nw) {
+                const int t = i / PARTS, b = i % PARTS * 16 + (lane >> 2), sub = lane & 3, e0 = 32 * b + 8 * sub;
+                const float *g = h + (size_t)t * E;
+                const float4 x0 = *reinterpret_cast<const float4 *>(g + e0), x1 = *reinterpret_cast<const float4 *>(g + e0 + 4);
+                const float4 w0 = *reinterpret_cast<const float4 *>(a.norm_w + e0),
+                             w1 = *reinterpret_cast<const float4 *>(a.norm_w + e0 + 4);
+                float gv[NS];
+#pragma unroll
+                for (int k = 0; k < NS; k++) gv[k] = g[L + 32 * k];
+                float acc = 0.0f;
+#pragma unroll
+                for (int k = 0; k < NS; k++) acc = fmaf(gv[k], gv[k], acc);
+                const float scale = rms_scale(acc, E, a.eps);
+                const float v[8] = {x0.x * (scale * w0.x), x0.y * (scale * w0.y), x0.z * (scale * w0.z), x0.w * (scale * w0.w),
+                                    x1.x * (scale * w1.x), x1.y * (scale * w1.y), x1.z * (scale * w1.z), x1.w * (scale * w1.w)};
+                float4 *o = reinterpret_cast<float4 *>(a.hn + (size_t)t * E + e0);
+                o[0] = make_float4(v[0], v[1], v[2], v[3]);
+                o[1] = make_float4(v[4], v[5], v[6], v[7]);
+                if (a.xq) quant_quad(v, E, t, b, sub, a);
+            }
+            return;
+        }
         for (int t = ((blockIdx.x - n_rw) * gridDim.y + blockIdx.y) * nhw + (threadIdx.x >> 5); t < T;
              t += nq * gridDim.y * nhw) {
             const float *g = h + (size_t)t * E;
@@ -321,7 +396,16 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     // the chains start once the tokens are in, the row's later words still
     // arriving
     __shared__ float xs[TC][E];
+    __shared__ __align__(16) float wns[ONE ? E : 4]; // the norm weights
     const int t0 = blockIdx.y * TC, nt = min(TC, T - t0);
+    if (ONE && a.norm_w) {
+        const unsigned dst = lds_addr(wns) + 16 * (threadIdx.x & ~(WAVE - 1));
+#pragma unroll
+        for (int c = 0; c < (E / 4 + NTH - 1) / NTH; c++) {
+            if (c * NTH + (int)(threadIdx.x & ~(WAVE - 1)) >= E / 4) break; // uniform over the wave
+            lds_dma16_at(a.norm_w + 4 * (c * NTH + threadIdx.x), dst + 16 * c * NTH);
+        }
+    }
     {
         constexpr int NP = TC * (E / 4) / NTH; // 16-byte pieces per thread
         const float4 *src = reinterpret_cast<const float4 *>(h + (size_t)t0 * E);
@@ -348,7 +432,7 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     // post_norm: this thread's norm weights
     constexpr int NWPT = E / NTH > 0 ? E / NTH : 1;
     float nw[NWPT];
-    if (a.norm_w) {
+    if (!ONE && a.norm_w) {
 #pragma unroll
         for (int j = 0; j < NWPT; j++) nw[j] = (int)threadIdx.x + NTH * j < E ? a.norm_w[threadIdx.x + NTH * j] : 0.0f;
     }
@@ -357,7 +441,29 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     __builtin_amdgcn_sched_barrier(0);
     wait_vm<NS / 4>();
     rm_barrier();
-    if (a.norm_w) {
+    if constexpr (ONE) {
+        if (a.norm_w) {
+            // the half wave's own copy of the token's chain elements gives
+            // the scale, then the normalised elements as the chain takes
+            // them: no further barrier
+            float v[NS];
+#pragma unroll
+            for (int k = 0; k < NS; k++) v[k] = xs[0][L + 32 * k];
+            float acc = 0.0f;
+#pragma unroll
+            for (int k = 0; k < NS; k++) acc = fmaf(v[k], v[k], acc);
+            const float scale = rms_scale(acc, E, a.eps);
+            acc = 0.0f;
+#pragma unroll
+            for (int k = 0; k < NS; k++) acc = fmaf(wv[k], v[k] * (scale * wns[L + 32 * k]), acc);
+            acc = half_tree32(acc); // valid in lane 0 of the half wave
+            if (valid && L == 0) {
+                if (row < n_expert) a.logits[(size_t)t0 * n_expert + row] = acc;
+                else a.glogit[t0] = acc;
+            }
+            return;
+        }
+    } else if (a.norm_w) {
         // rms_norm of the staged tokens in place: a half wave per token forms
         // the scale, then every thread scales its elements, v * (scale * w)
         __shared__ float scl[TC];
@@ -2875,7 +2981,8 @@ hipError_t launch_router(const RouterArgs &a0, hipStream_t st)
     }
     const int rows = a.n_expert + 1;
     // quantisation workgroups beside the row groups: about one block per thread
-    const int qblocks = a.xq || a.norm_w ? a.T * (a.E / 32) : 0;
+    // (with the post_norm and few tokens a wave per 16 of them, four lanes a block)
+    const int qblocks = (a.xq || a.norm_w ? a.T * (a.E / 32) : 0) * (a.norm_w && a.T <= ROUTER_FEW_T ? 4 : 1);
     // 8 rows per workgroup; tokens split over grid.y in chunks of TC (32 KB of
     // LDS, 64 KB past 2 TC tokens); batches of 2..64 tokens in chunks of TC / 4
     // (up to 16 tokens) or TC / 2: more workgroups, shorter chains each
