@@ -347,18 +347,44 @@ int dense_scratch_fit(biv_hip_ctx *ctx, const biv_hip_dense *d, int T)
     return 0;
 }
 
-// Whether a half of the dense FFN (T rows against a matrix of rows x K) runs
-// on the matrix cores (launch_exact) or in the chain matvecs (launch_long_mv).
-// The matvecs' time grows with the tokens, the matrix-core kernel's up to 16
-// tokens is the latency of its K steps: layers of 4096 x 12288 cross between
-// 5 and 6 tokens (Q8_0 at 6 / 8 / 16: 87 / 88 / 93 against 90 / 105 / 150 us;
-// Q4_K/Q6_K at 5 / 8 / 16: 101 / 102 / 108 against 118 / 186 / 318), small
-// Q8_0 layers later (1024 x 1536 at 20 / 40: 27 / 27 against 22 / 29; 2048 x
-// 3584 at 8 / 12: 31 / 32 against 30 / 34; 1536 x 7680 at 7: 43 against 44).
-bool dense_exact(int ty, int T, int rows, int K)
+// Whether a half of the dense FFN (T rows against a matrix of rows x K; gate
+// and up together, or down) runs on the matrix cores (launch_exact) or in the
+// chain matvecs (launch_long_mv).
+//
+// Up to 16 tokens the matrix-core kernel's time is the latency of its K steps,
+// whatever T and rows are.  The matvecs' (8 tokens a workgroup past 5; fewer
+// have instances of their own width) is such a latency too while their
+// T * rows / 16 (gate/up) or / 32 (down) waves are few against the 1024 SIMDs,
+// then grows with T * rows.  So the line is one of T * rows, K on both sides.
+// Measured over layers of 512 to 5120 x 512 to 17408, weights cold where 24
+// layers of that shape would be; time of the half on the matrix cores minus
+// that in the matvecs, us:
+//   Q8_0 gate/up  rows 12288 T = 5 / 6: -4 / -18 of 76; 4096 (K = 4096) T = 7
+//     / 8 / 9: 1.8 / 0.6 / -5 of 40; 3584 T = 8 / 9: -0.2 / -0.8; 1536 T = 16
+//     / 17 / 24: 0.1 / 3 / -4; 512 T = 24 / 64 / 80: 0.9 / 0.1 / -3.5
+//   Q8_0 down     rows 4096 (K = 8192) T = 8 / 16 / 20 / 24: 7 / 5 / 2 / -7 of
+//     76; 3072 T = 20 / 24: 6 / -4; 2048 (K = 8192) T = 33 / 36 / 40: 10 / 3 /
+//     -6; 1024 T = 65 / 72: 6 / -0.6; 512 T = 128 / 144 / 200: 8 / 0.1 / -4
+//   Q6_K gate/up  rows 12288 T = 5 / 6: 4 / -13; 4096 T = 6 / 7: 3 / -0.2;
+//     3584 T = 7 / 8: -0.4 / -1.8; 1536 T = 17 / 20: 0.9 / -0.8; 512 T = 33 /
+//     64 / 72: 0.9 / -0.3 / -4
+//   Q6_K down     rows 4096 (K = 8192) T = 8 / 9: 5 / -4; 3072 T = 9 / 12: 6 /
+//     -7; 2048 T = 17 / 20: 4 / -0.7; 1024 T = 33 / 36: 5 / 0.1; 512 T = 64 /
+//     72: 10 / -9.  Rows too long for the matvecs' LDS (11264 on; then two
+//     chunks at a time there) later: K = 12288, rows 4096 T = 12 / 16 / 20: 14 /
+//     0.1 / -14; 3072 T = 18 / 20: 13 / -7; 2048 T = 32 / 40: 13 / -30
+//   Q4_K (two FMAs and the mins a word on either side) from four tokens:
+//     gate/up 12288 x 4096 T = 2 / 3 / 4: -9 / -23 / -35 of 128; 4096 x 1024
+//     1.3 / 0 / -1.9; 1536 x 2048 4.5 / 2.7 / -0.2; down 4096 x 8192 10 / 5 /
+//     -1.5; 1024 x 4096 5 / 0.6 / -5.5; at 17 to 200 tokens -2.5 and more
+bool dense_exact(int ty, bool gateup, int T, int rows, int K)
 {
-    if (ty == biv::T_BF16 || T < 7) return false;
-    return ty != biv::T_Q8_0 || (size_t)T * rows * K >= ((size_t)72 << 20);
+    const size_t n = (size_t)T * rows;
+    if (ty == biv::T_Q4K) return T >= 4;
+    if (T < 6) return false;
+    if (ty == biv::T_Q8_0) return n >= (gateup ? 32 : 72) * 1024;
+    if (ty == biv::T_Q6K) return n >= (gateup ? 28 : K < 11 * 1024 ? 36 : 60) * 1024;
+    return false; // BF16
 }
 
 // dense_ffn (model.rs:1118-1126) of T rows on the context's stream:
@@ -378,7 +404,7 @@ int dense_forward(biv_hip_ctx *ctx, const biv_hip_dense *d, const float *h, int 
     auto half = [&](const DevMat &A, const DevMat *B, const float *in, int K, int8_t *q, float *qd, float *qs,
                     float *dst, int add, const char *what) -> int {
         const int n_blocks = T * (K / 32);
-        if (dense_exact(A.ty, T, A.rows, K)) {
+        if (dense_exact(A.ty, B != nullptr, T, A.rows, K)) {
             biv::ExactArgs e{};
             e.a = A;
             if (B) e.b = *B;

@@ -68,6 +68,21 @@ def test_exact_64(orc, engine, types, n_embd, n_ff, tokens):
     run(orc, engine, types, n_embd, n_ff, tokens)
 
 
+# The edges of the rule that takes a half of the layer here (a matrix-core half
+# beside a matvec one among them): the first token counts of Q4_K, and with
+# 5120 rows on one side every tile of Q8_0's and Q6_K's gate/up and down from
+# the first counts on
+@pytest.mark.parametrize("types,n_embd,n_ff,tokens", [
+    ((Q4K, Q4K, Q4K), 1024, 1536, (3, 4, 5, 6, 15, 17, 33)),
+    ((Q8_0, Q8_0, Q8_0), 512, 5120, (5, 6, 7, 15, 17, 33, 49)),
+    ((Q8_0, Q8_0, Q8_0), 5120, 1536, (14, 15, 16, 17, 32, 33, 49)),
+    ((Q6K, Q6K, Q6K), 512, 5120, (5, 6, 16, 17, 33, 49)),
+    ((Q6K, Q6K, Q6K), 5120, 1536, (7, 8, 16, 17, 33, 49)),
+])
+def test_exact_edges(orc, engine, types, n_embd, n_ff, tokens):
+    run(orc, engine, types, n_embd, n_ff, tokens)
+
+
 @pytest.mark.parametrize("types,T", [((Q8_0, Q8_0, Q8_0), 40), ((Q4K, Q4K, Q6K), 20)])
 def test_exact_special_rows(orc, engine, types, T):
     """Rows of zeros, of huge and tiny values, and with an infinity or a NaN,
