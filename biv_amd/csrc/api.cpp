@@ -48,6 +48,7 @@ struct DenseScratch {
     int8_t *xq = nullptr, *aq = nullptr;
     float *xd = nullptr, *xs = nullptr, *act = nullptr, *ad = nullptr, *as = nullptr;
     float *h_stage = nullptr, *o_stage = nullptr;
+    bool f16 = false; // xq and aq hold f16 quants (else int8 only)
 };
 
 // Device buffers of one forward, grown to the largest T seen.
@@ -125,6 +126,14 @@ int hip_fail(biv_hip_ctx *ctx, hipError_t e, const char *what)
     return fail(ctx, BIV_HIP_E_DEVICE, "%s: %s", what, hipGetErrorString(e));
 }
 
+// a refused hipMalloc; its error is taken off the thread, or the next
+// launch's check would report it
+int no_mem(biv_hip_ctx *ctx, const char *what, size_t bytes, hipError_t e)
+{
+    (void)hipGetLastError();
+    return fail(ctx, BIV_HIP_E_NOMEM, "%s(%zu): %s", what, bytes, hipGetErrorString(e));
+}
+
 #define HIP_TRY(ctx, call, what)                                                                                \
     do {                                                                                                        \
         hipError_t e_ = (call);                                                                                 \
@@ -154,7 +163,7 @@ int dev_alloc(biv_hip_ctx *ctx, size_t bytes, uint8_t **out)
 {
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
-    if (e != hipSuccess) return fail(ctx, BIV_HIP_E_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess) return no_mem(ctx, "hipMalloc", bytes, e);
     ctx->allocs.push_back(p);
     ctx->bytes += bytes;
     *out = static_cast<uint8_t *>(p);
@@ -304,8 +313,7 @@ template <class T> int sc_alloc(biv_hip_ctx *ctx, size_t count, T **out, std::ve
 {
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, count * sizeof(T) + 16);
-    if (e != hipSuccess)
-        return fail(ctx, BIV_HIP_E_NOMEM, "scratch hipMalloc(%zu): %s", count * sizeof(T), hipGetErrorString(e));
+    if (e != hipSuccess) return no_mem(ctx, "scratch hipMalloc", count * sizeof(T), e);
     (bufs ? bufs : &ctx->sc.bufs)->push_back(p);
     *out = static_cast<T *>(p);
     return 0;
@@ -317,26 +325,32 @@ void dense_scratch_free(biv_hip_ctx *ctx)
     ctx->dsc = DenseScratch{};
 }
 
-// Make the dense scratch fit T rows of a layer of E x ff.
+// Make the dense scratch fit T rows of a layer of E x ff.  The quants have
+// room for f16, which the matrix-core kernel takes; where that does not fit
+// the device any more, for int8, and the layer runs in the matvecs.
 int dense_scratch_fit(biv_hip_ctx *ctx, const biv_hip_dense *d, int T)
 {
     DenseScratch &s = ctx->dsc;
     if (T <= s.cap_T && d->E <= s.E && d->ff <= s.ff) return 0;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream), "sync");
     const int cap = std::max(T, std::max(s.cap_T, 8)), E = std::max(d->E, s.E), ff = std::max(d->ff, s.ff);
-    dense_scratch_free(ctx);
     const size_t Tc = cap;
     auto *b = &s.bufs;
     int rc = 0;
-    rc = rc ? rc : sc_alloc(ctx, Tc * E * 2, &s.xq, b); // int8 or f16 quants
-    rc = rc ? rc : sc_alloc(ctx, Tc * E / 32, &s.xd, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * E / 32, &s.xs, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * ff, &s.act, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * ff * 2, &s.aq, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * ff / 32, &s.ad, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * ff / 32, &s.as, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * E, &s.h_stage, b);
-    rc = rc ? rc : sc_alloc(ctx, Tc * E, &s.o_stage, b);
+    for (int width = 2; width >= 1; width--) { // bytes of a quant
+        dense_scratch_free(ctx);
+        rc = sc_alloc(ctx, Tc * E * width, &s.xq, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * E / 32, &s.xd, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * E / 32, &s.xs, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * ff, &s.act, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * ff * width, &s.aq, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * ff / 32, &s.ad, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * ff / 32, &s.as, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * E, &s.h_stage, b);
+        rc = rc ? rc : sc_alloc(ctx, Tc * E, &s.o_stage, b);
+        s.f16 = width == 2;
+        if (rc != BIV_HIP_E_NOMEM) break;
+    }
     if (rc) {
         dense_scratch_free(ctx);
         return rc;
@@ -404,7 +418,7 @@ int dense_forward(biv_hip_ctx *ctx, const biv_hip_dense *d, const float *h, int 
     auto half = [&](const DevMat &A, const DevMat *B, const float *in, int K, int8_t *q, float *qd, float *qs,
                     float *dst, int add, const char *what) -> int {
         const int n_blocks = T * (K / 32);
-        if (dense_exact(A.ty, B != nullptr, T, A.rows, K)) {
+        if (s.f16 && dense_exact(A.ty, B != nullptr, T, A.rows, K)) {
             biv::ExactArgs e{};
             e.a = A;
             if (B) e.b = *B;
@@ -1139,8 +1153,7 @@ int biv_hip_malloc(biv_hip_ctx *ctx, size_t bytes, void **out)
     if (!ctx || !out) return BIV_HIP_E_INVALID;
     HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
     hipError_t e = hipMalloc(out, bytes ? bytes : 1);
-    if (e != hipSuccess) return fail(ctx, BIV_HIP_E_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-    return 0;
+    return e == hipSuccess ? 0 : no_mem(ctx, "hipMalloc", bytes, e);
 }
 
 int biv_hip_free(biv_hip_ctx *ctx, void *p)

@@ -98,3 +98,58 @@ def test_exact_special_rows(orc, engine, types, T):
             h[5, 7] = np.nan
     with np.errstate(all="ignore"):
         run(orc, engine, types, 2048, 1536, (T,), edit)
+
+
+def test_scratch_limit(orc):
+    """Where the f16 quants no longer fit the device and int8 ones do, the
+    layer runs in the matvecs: the same bits, and nothing is left behind by the
+    refused allocations; where neither fits, an error, after which smaller
+    calls work."""
+    from biv_amd import hip
+    E = ff = 512
+    T = 100_000
+    f16 = T * (10 * E + 6 * ff + (E + ff) // 4)  # bytes of scratch
+    int8 = f16 - T * (E + ff)
+    layer = synth.make_dense(23, n_embd=E, n_ff=ff, types=(Q4K, Q4K, Q4K))
+    h = synth.make_tokens(5, T, n_embd=E)
+    outs = {}
+    for room in (None, (f16 + int8) // 2, int8 // 2):
+        with hip.HipEngine(0) as e, hip.HipEngine(0) as filler:
+            d = e.dense(layer)
+            hd, od = e.malloc(h.nbytes), e.malloc(h.nbytes)
+            e.h2d(hd, h)
+            d.forward_device(hd, 1, od)  # (code is loaded before the room is taken)
+            e.sync()
+            held = []
+            if room:
+                hole, size = filler.malloc(room), 8 << 30
+                while size >= 8 << 20:
+                    try:
+                        held.append(filler.malloc(size))
+                    except hip.HipError as err:
+                        assert err.code == -4
+                        size >>= 1
+                filler.free(hole)
+            print(f"case scratch_limit room={room} fills={len(held)}", flush=True)
+            try:
+                if room and room < int8:
+                    with pytest.raises(hip.HipError) as err:
+                        d.forward_device(hd, T, od)
+                    assert err.value.code == -4
+                    d.forward_device(hd, 40, od)
+                else:
+                    d.forward_device(hd, T, od)
+                e.sync()
+                outs[room] = e.d2h(np.empty_like(h), od)
+            finally:
+                for p in held:
+                    filler.free(p)
+                e.free(hd)
+                e.free(od)
+    full, mid, small = outs.values()
+    assert np.array_equal(full.view(np.uint32), mid.view(np.uint32))
+    assert np.array_equal(full[:40].view(np.uint32), small[:40].view(np.uint32))
+    rows = [0, 1, 7, 8, T // 2, T - 1]
+    g, u, dn = layer.gate, layer.up, layer.down
+    ref = orc.dense_ffn(g.ty, g.data, u.ty, u.data, dn.ty, dn.data, E, ff, h[rows], threads=8)
+    assert np.array_equal(ref.view(np.uint32), full[rows].view(np.uint32))
