@@ -399,11 +399,16 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     __shared__ __align__(16) float wns[ONE ? E : 4]; // the norm weights
     const int t0 = blockIdx.y * TC, nt = min(TC, T - t0);
     if (ONE && a.norm_w) {
-        const unsigned dst = lds_addr(wns) + 16 * (threadIdx.x & ~(WAVE - 1));
+        const unsigned wave0 = threadIdx.x & ~(WAVE - 1);
+        if ((uintptr_t)a.norm_w & 15) { // any float address: a float a lane
+            for (unsigned c = wave0; c < E; c += NTH)
+                lds_dma4_at(a.norm_w + c + (threadIdx.x & (WAVE - 1)), lds_addr(wns) + 4 * c);
+        } else {
 #pragma unroll
-        for (int c = 0; c < (E / 4 + NTH - 1) / NTH; c++) {
-            if (c * NTH + (int)(threadIdx.x & ~(WAVE - 1)) >= E / 4) break; // uniform over the wave
-            lds_dma16_at(a.norm_w + 4 * (c * NTH + threadIdx.x), dst + 16 * c * NTH);
+            for (int c = 0; c < (E / 4 + NTH - 1) / NTH; c++) {
+                if (c * NTH + (int)wave0 >= E / 4) break; // uniform over the wave
+                lds_dma16_at(a.norm_w + 4 * (c * NTH + threadIdx.x), lds_addr(wns) + 16 * (wave0 + c * NTH));
+            }
         }
     }
     {

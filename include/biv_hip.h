@@ -219,8 +219,8 @@ int biv_hip_rms_norm(biv_hip_ctx *ctx, float *x_dev, const float *w_dev, int row
  * (engine/src/model.rs:788-790), in device memory: h = rms_norm(x, norm, eps)
  * (ops::rms_norm_into), then x += moe(h) (ops::add_inplace), for the n rows of
  * x (n x n_embd floats).  norm_dev holds the layer's post_norm (n_embd
- * floats).  h lives in the context's scratch.  Queued on the context's
- * stream. */
+ * floats, at any float's address).  h lives in the context's scratch.  Queued
+ * on the context's stream. */
 int biv_hip_moe_ffn_step(biv_hip_ctx *ctx, const biv_hip_moe *moe, float *x_dev, const float *norm_dev, float eps,
                          int n);
 

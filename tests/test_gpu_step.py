@@ -1,0 +1,53 @@
+"""biv_hip_moe_ffn_step, x += moe(rms_norm(x)), below 64 tokens against the
+oracle, at every width, on both sides of the router launch's switch at 16/17
+tokens.  Every sum runs in the reference's order, so the bound is equality."""
+import numpy as np
+import pytest
+
+from biv_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+Q8_0, Q4K, Q6K = synth.Q8_0, synth.Q4K, synth.Q6K
+EPS = 1e-6
+
+
+@pytest.fixture(scope="module")
+def engine():
+    from biv_amd import hip
+    e = hip.HipEngine(0)
+    yield e
+    e.close()
+
+
+def inputs(n_embd, T):
+    rng = np.random.default_rng(400 + T)
+    w = (1.0 + 0.05 * rng.standard_normal(n_embd)).astype(np.float32)
+    x = np.float32(3.0) * synth.make_tokens(500 + T, T, n_embd=n_embd, offsets=T > 1)
+    return x, w
+
+
+def step(engine, moe, x, w, shift=0):
+    """The step with the norm weights `shift` floats into their buffer."""
+    xd, nd = engine.malloc(x.nbytes), engine.malloc(w.nbytes + 16)
+    try:
+        engine.h2d(xd, x)
+        engine.h2d(nd + 4 * shift, w)
+        moe.ffn_step_device(xd, nd + 4 * shift, EPS, x.shape[0])
+        return engine.d2h(np.empty_like(x), xd)
+    finally:
+        engine.free(xd)
+        engine.free(nd)
+
+
+@pytest.mark.parametrize("n_embd", [512, 1024, 2048])
+def test_norm_alignment(engine, n_embd):
+    """The norm weights at any float's address give the bits that they give
+    at an aligned one."""
+    moe = engine.moe(synth.make_layer(41, n_embd=n_embd, n_expert=8, k=2, n_ff=512, n_ff_sh=512))
+    for T in (1, 5, 16, 17):
+        x, w = inputs(n_embd, T)
+        ref = step(engine, moe, x, w)
+        for shift in (1, 2, 3):
+            print(f"case norm_alignment {n_embd} T={T} shift={shift}", flush=True)
+            assert np.array_equal(ref.view(np.uint32), step(engine, moe, x, w, shift).view(np.uint32))
