@@ -171,10 +171,10 @@ __device__ inline void quant_block_lds(const float4 *v, int K, int b, int *qrow,
     if (srow) srow[sb] = db * (float)sum;
 }
 
-__device__ inline void quant_block(const float (&v)[32], int K, size_t row, int b, int8_t *qs, float *d, float *s,
-                                   bool f16 = false)
+template <bool F16 = false>
+__device__ inline void quant_block(const float (&v)[32], int K, size_t row, int b, int8_t *qs, float *d, float *s)
 {
-    if (f16)
+    if constexpr (F16)
         return quant_block_f16(v, b, reinterpret_cast<uint2 *>(qs + row * K * 2), d + row * (K / 32), s + row * (K / 32));
     quant_block_at(v, K, b, reinterpret_cast<int *>(qs + row * K), d + row * (K / 32), s + row * (K / 32));
 }
@@ -284,21 +284,27 @@ __device__ inline void quant_quad(const float (&v)[8], int E, int t, int b, int 
     sum += __builtin_amdgcn_mov_dpp(sum, 0xB1, 0xF, 0xF, true);
     sum += __builtin_amdgcn_mov_dpp(sum, 0x4E, 0xF, 0xF, true);
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        if (a.f16) reinterpret_cast<uint2 *>(a.xq + (size_t)t * E * 2)[f16_word(b, 2 * sub + j)] = i8x4_to_f16x4(w[j]);
-        else reinterpret_cast<int *>(a.xq + (size_t)t * E)[lay::q8_word(b, 2 * sub + j)] = (int)w[j];
-    }
+    for (int j = 0; j < 2; j++)
+        reinterpret_cast<int *>(a.xq + (size_t)t * E)[lay::q8_word(b, 2 * sub + j)] = (int)w[j];
     if (sub == 0) {
-        const size_t o = (size_t)t * (E / 32) + (a.f16 ? b : lay::q8_scale(E, b));
+        const size_t o = (size_t)t * (E / 32) + lay::q8_scale(E, b);
         a.xd[o] = db;
         a.xs[o] = db * (float)sum;
     }
 }
 
-template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void k_router(RouterArgs a)
+// What a k_router instance does before the logits: nothing, or the post_norm
+// (norm_w), for few tokens or many; and whether h is quantised as f16 (F16).
+// Compiled apart: in one kernel the few-token norm's registers were every
+// caller's (2048 wide, 256 threads: 140 VGPRs, 3 waves a SIMD, against 95 and 5
+// without it; layers of 64 experts at 2 to 16 tokens 0.5-0.9% slower, the step
+// at 17 and 40 tokens 1%, at 1 token 16.9 against 16.4 us).
+enum { NORM_NONE, NORM_FEW, NORM_MANY };
+
+template <int NS, int TC, int NORM, bool F16, int NTH> __global__ __launch_bounds__(NTH) void k_router(RouterArgs a)
 {
-    // one token a workgroup (the 64-thread instances serve one token only)
-    constexpr bool ONE = TC == 1 || NTH == 64;
+    // few tokens, one a workgroup (the 64-thread instances serve one token only)
+    constexpr bool ONE = NORM == NORM_FEW && (TC == 1 || NTH == 64);
     constexpr int RPW = NTH / 32; // rows per workgroup (a half wave each)
     constexpr int E = 32 * NS;
     const float *__restrict__ router = a.router;
@@ -309,13 +315,11 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     // xq (BF16 layers, which read h as f32) there are none, or, with the
     // post_norm, they write hn only.
     const int n_rw = (n_expert + 1 + RPW - 1) / RPW;
-    if ((int)blockIdx.x >= n_rw && a.norm_w) {
-        // post_norm first: a half wave per token forms its RMS scale (the
-        // row in registers), then quantises the normalised row, two blocks
-        // per lane, and writes it to hn
+    if (NORM != NORM_NONE && (int)blockIdx.x >= n_rw) {
+        // post_norm first; the normalised rows go to hn too
         const int L = threadIdx.x & 31, nhw = NTH / 32;
         const int nq = gridDim.x - n_rw;
-        if (T <= ROUTER_FEW_T) {
+        if constexpr (NORM == NORM_FEW) {
             // Few tokens: a wave per 16 blocks of a token, 4 lanes to a block
             // (8 elements each), every load issued before the chain; each of
             // a token's waves forms the scale for itself.  (A half wave per
@@ -346,6 +350,8 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
             }
             return;
         }
+        // Many: a half wave per token forms its RMS scale (the row in
+        // registers), then quantises the normalised row, two blocks per lane
         for (int t = ((blockIdx.x - n_rw) * gridDim.y + blockIdx.y) * nhw + (threadIdx.x >> 5); t < T;
              t += nq * gridDim.y * nhw) {
             const float *g = h + (size_t)t * E;
@@ -370,7 +376,7 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
                     v[4 * j + 3] = v[4 * j + 3] * (scale * w.w);
                     o4[j] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
                 }
-                if (a.xq) quant_block(v, E, t, b, a.xq, a.xd, a.xs, a.f16);
+                if (a.xq) quant_block<F16>(v, E, t, b, a.xq, a.xd, a.xs);
             }
         }
         return;
@@ -381,7 +387,7 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
              i += nthreads) {
             float v[32];
             load32(h + 32 * (size_t)i, v);
-            quant_block(v, E, i / (E / 32), i % (E / 32), a.xq, a.xd, a.xs, a.f16);
+            quant_block<F16>(v, E, i / (E / 32), i % (E / 32), a.xq, a.xd, a.xs);
         }
         return;
     }
@@ -398,7 +404,7 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     __shared__ float xs[TC][E];
     __shared__ __align__(16) float wns[ONE ? E : 4]; // the norm weights
     const int t0 = blockIdx.y * TC, nt = min(TC, T - t0);
-    if (ONE && a.norm_w) {
+    if (ONE) {
         const unsigned wave0 = threadIdx.x & ~(WAVE - 1);
         if ((uintptr_t)a.norm_w & 15) { // any float address: a float a lane
             for (unsigned c = wave0; c < E; c += NTH)
@@ -437,7 +443,7 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     // post_norm: this thread's norm weights
     constexpr int NWPT = E / NTH > 0 ? E / NTH : 1;
     float nw[NWPT];
-    if (!ONE && a.norm_w) {
+    if (NORM != NORM_NONE && !ONE) {
 #pragma unroll
         for (int j = 0; j < NWPT; j++) nw[j] = (int)threadIdx.x + NTH * j < E ? a.norm_w[threadIdx.x + NTH * j] : 0.0f;
     }
@@ -447,28 +453,26 @@ template <int NS, int TC, int NTH = 256> __global__ __launch_bounds__(NTH) void 
     wait_vm<NS / 4>();
     rm_barrier();
     if constexpr (ONE) {
-        if (a.norm_w) {
-            // the half wave's own copy of the token's chain elements gives
-            // the scale, then the normalised elements as the chain takes
-            // them: no further barrier
-            float v[NS];
+        // the half wave's own copy of the token's chain elements gives the
+        // scale, then the normalised elements as the chain takes them: no
+        // further barrier
+        float v[NS];
 #pragma unroll
-            for (int k = 0; k < NS; k++) v[k] = xs[0][L + 32 * k];
-            float acc = 0.0f;
+        for (int k = 0; k < NS; k++) v[k] = xs[0][L + 32 * k];
+        float acc = 0.0f;
 #pragma unroll
-            for (int k = 0; k < NS; k++) acc = fmaf(v[k], v[k], acc);
-            const float scale = rms_scale(acc, E, a.eps);
-            acc = 0.0f;
+        for (int k = 0; k < NS; k++) acc = fmaf(v[k], v[k], acc);
+        const float scale = rms_scale(acc, E, a.eps);
+        acc = 0.0f;
 #pragma unroll
-            for (int k = 0; k < NS; k++) acc = fmaf(wv[k], v[k] * (scale * wns[L + 32 * k]), acc);
-            acc = half_tree32(acc); // valid in lane 0 of the half wave
-            if (valid && L == 0) {
-                if (row < n_expert) a.logits[(size_t)t0 * n_expert + row] = acc;
-                else a.glogit[t0] = acc;
-            }
-            return;
+        for (int k = 0; k < NS; k++) acc = fmaf(wv[k], v[k] * (scale * wns[L + 32 * k]), acc);
+        acc = half_tree32(acc); // valid in lane 0 of the half wave
+        if (valid && L == 0) {
+            if (row < n_expert) a.logits[(size_t)t0 * n_expert + row] = acc;
+            else a.glogit[t0] = acc;
         }
-    } else if (a.norm_w) {
+        return;
+    } else if constexpr (NORM != NORM_NONE) {
         // rms_norm of the staged tokens in place: a half wave per token forms
         // the scale, then every thread scales its elements, v * (scale * w)
         __shared__ float scl[TC];
@@ -2955,10 +2959,23 @@ hipError_t launch_rms_norm(const float *x, float *y, const float *w, int rows, i
 }
 
 // threads of a router workgroup for a single token (two rows each)
-#ifndef BIV_ROUTER_T1_NTH
-#define BIV_ROUTER_T1_NTH 64
-#endif
+constexpr int ROUTER_T1_NTH = 64;
 int prep_min_t() { return RT_MIN_T; }
+
+// k_router over workgroups of NTH / 32 rows and TC tokens, with NORM where
+// the call has a post_norm
+template <int NS, int TC, int NORM, bool F16, int NTH = 256>
+static hipError_t launch_router_n(const RouterArgs &a, hipStream_t st)
+{
+    // quantisation workgroups beside the row groups: about one block per thread
+    // (with NORM_FEW a wave per 16 of them, four lanes a block)
+    const int qblocks = (a.xq || a.norm_w ? a.T * (a.E / 32) : 0) * (a.norm_w && NORM == NORM_FEW ? 4 : 1);
+    const int gy = (a.T + TC - 1) / TC, rows = a.n_expert + 1;
+    const dim3 grid((rows + NTH / 32 - 1) / (NTH / 32) + (qblocks + NTH * gy - 1) / (NTH * gy), gy);
+    if (a.norm_w) k_router<NS, TC, NORM, F16, NTH><<<grid, NTH, 0, st>>>(a);
+    else k_router<NS, TC, NORM_NONE, F16, NTH><<<grid, NTH, 0, st>>>(a);
+    return hipGetLastError();
+}
 
 hipError_t launch_router(const RouterArgs &a0, hipStream_t st)
 {
@@ -2984,34 +3001,18 @@ hipError_t launch_router(const RouterArgs &a0, hipStream_t st)
 #undef BIV_RM_LAUNCH
         return hipGetLastError();
     }
-    const int rows = a.n_expert + 1;
-    // quantisation workgroups beside the row groups: about one block per thread
-    // (with the post_norm and few tokens a wave per 16 of them, four lanes a block)
-    const int qblocks = (a.xq || a.norm_w ? a.T * (a.E / 32) : 0) * (a.norm_w && a.T <= ROUTER_FEW_T ? 4 : 1);
-    // 8 rows per workgroup; tokens split over grid.y in chunks of TC (32 KB of
-    // LDS, 64 KB past 2 TC tokens); batches of 2..64 tokens in chunks of TC / 4
-    // (up to 16 tokens) or TC / 2: more workgroups, shorter chains each
+    // 8 rows per workgroup (2 for one token); tokens split over grid.y in chunks
+    // of 2 TC (64 KB of LDS); batches of 2..64 tokens in chunks of TC / 4 (up
+    // to 16 tokens) or TC / 2: more workgroups, shorter chains each
 #define BIV_ROUTER_CASE(NS)                                                                                     \
     if (a.E == 32 * NS) {                                                                                       \
         constexpr int TC = 8192 / (32 * NS);                                                                    \
-        if (a.T > 1 && a.T <= 64) {                                                                             \
-            /* small batches: one or two tokens per workgroup, more workgroups */                               \
-            constexpr int TS1 = TC / 4 > 0 ? TC / 4 : 1, TS2 = TC / 2 > 0 ? TC / 2 : 1;                         \
-            const int ts = a.T <= 16 ? TS1 : TS2, gy = (a.T + ts - 1) / ts;                                     \
-            const dim3 grid((rows + 7) / 8 + (qblocks + 256 * gy - 1) / (256 * gy), gy);                        \
-            if (ts == TS1) k_router<NS, TS1><<<grid, 256, 0, st>>>(a);                                          \
-            else k_router<NS, TS2><<<grid, 256, 0, st>>>(a);                                                    \
-        } else if (a.T == 1 && BIV_ROUTER_T1_NTH != 256) {                                                      \
-            constexpr int N1 = BIV_ROUTER_T1_NTH;                                                               \
-            k_router<NS, TC, N1><<<dim3((rows + N1 / 32 - 1) / (N1 / 32) + (qblocks + N1 - 1) / N1, 1), N1, 0, st>>>(a); \
-        } else if (a.T <= 2 * TC) {                                                                             \
-            const int gy = (a.T + TC - 1) / TC;                                                                 \
-            k_router<NS, TC><<<dim3((rows + 7) / 8 + (qblocks + 256 * gy - 1) / (256 * gy), gy), 256, 0, st>>>(a); \
-        } else {                                                                                                \
-            const int gy = (a.T + 2 * TC - 1) / (2 * TC);                                                       \
-            k_router<NS, 2 * TC><<<dim3((rows + 7) / 8 + (qblocks + 256 * gy - 1) / (256 * gy), gy), 256, 0, st>>>(a); \
-        }                                                                                                       \
-        return hipGetLastError();                                                                               \
+        if (a.f16 && a.T <= 64) return launch_router_n<NS, TC / 2, NORM_MANY, true>(a, st);                     \
+        if (a.f16) return launch_router_n<NS, 2 * TC, NORM_MANY, true>(a, st);                                  \
+        if (a.T == 1) return launch_router_n<NS, TC, NORM_FEW, false, ROUTER_T1_NTH>(a, st);                    \
+        if (a.T <= ROUTER_FEW_T) return launch_router_n<NS, TC / 4, NORM_FEW, false>(a, st);                    \
+        if (a.T <= 64) return launch_router_n<NS, TC / 2, NORM_MANY, false>(a, st);                             \
+        return launch_router_n<NS, 2 * TC, NORM_MANY, false>(a, st);                                            \
     }
     BIV_ROUTER_CASE(64)
     BIV_ROUTER_CASE(32)
