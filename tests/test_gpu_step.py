@@ -1,6 +1,8 @@
-"""biv_hip_moe_ffn_step, x += moe(rms_norm(x)), below 64 tokens against the
-oracle, at every width, on both sides of the router launch's switch at 16/17
-tokens.  Every sum runs in the reference's order, so the bound is equality."""
+"""biv_hip_moe_ffn_step, x += moe(rms_norm(x)), against the oracle at every
+width: on both sides of the router launch's switch at 16/17 tokens, and with
+the f16 quants of 64 tokens and up, to 256, where the pre-pass takes over.
+Every sum runs in the reference's order (from 64 tokens with a Q4_K down, which
+stays on the chain kernels), so the bound is equality."""
 import numpy as np
 import pytest
 
@@ -8,7 +10,7 @@ from biv_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-Q8_0, Q4K, Q6K = synth.Q8_0, synth.Q4K, synth.Q6K
+Q8_0, Q4K, Q6K, BF16 = synth.Q8_0, synth.Q4K, synth.Q6K, synth.BF16
 EPS = 1e-6
 
 
@@ -51,3 +53,29 @@ def test_norm_alignment(engine, n_embd):
         for shift in (1, 2, 3):
             print(f"case norm_alignment {n_embd} T={T} shift={shift}", flush=True)
             assert np.array_equal(ref.view(np.uint32), step(engine, moe, x, w, shift).view(np.uint32))
+
+
+def against_oracle(orc, engine, layer, n_embd, tokens):
+    moe = engine.moe(layer)
+    for T in tokens:
+        print(f"case step {n_embd} T={T}", flush=True)
+        x, w = inputs(n_embd, T)
+        ref = x + orc.moe(layer, orc.rms_norm(x, w, EPS), threads=8)
+        got = step(engine, moe, x, w)
+        assert np.array_equal(ref.view(np.uint32), got.view(np.uint32)), np.mean(ref != got)
+
+
+# 20 experts (and the gate row): the last row groups of a router launch are partial
+@pytest.mark.parametrize("n_embd", [512, 1024, 2048])
+@pytest.mark.parametrize("types", [(Q8_0, Q8_0, Q8_0), (Q4K, Q4K, Q6K), (BF16, BF16, BF16)])
+@pytest.mark.parametrize("shared", [True, False])
+def test_step_few_tokens(orc, engine, n_embd, types, shared):
+    layer = synth.make_layer(42, n_embd=n_embd, n_expert=20, k=4, types=types, shared=shared)
+    against_oracle(orc, engine, layer, n_embd, (1, 2, 3, 4, 6, 15, 16, 17, 33))
+
+
+@pytest.mark.parametrize("n_embd", [512, 1024, 2048])
+@pytest.mark.parametrize("types", [(Q8_0, Q8_0, Q4K), (Q4K, Q4K, Q4K)])
+def test_step_f16_quants(orc, engine, n_embd, types):
+    layer = synth.make_layer(43, n_embd=n_embd, n_expert=20, k=4, types=types)
+    against_oracle(orc, engine, layer, n_embd, (64, 65, 255, 256))
