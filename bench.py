@@ -4,8 +4,8 @@
 A step is one forward of one MoE layer (router, routing, dispatch, grouped
 Q8_0 expert SwiGLU, shared expert, combine) over T tokens already resident in
 HBM.  The headline workload is the decode-verify configuration (T = 5: one
-token plus four MTP drafts); T = 1, 40 and the
-T = 512 Zipf-skewed prefill chunk are reported in `sweep`.
+token plus four MTP drafts); T = 1, 40 and the T = 512 Zipf-skewed prefill
+chunk are reported in `sweep`.
 
 Steps rotate over `--layers` distinct copies of the layer in HBM (16 x 856 MB
 by default), so the expert weights a step reads are not left in the 256 MB
@@ -199,11 +199,10 @@ def bench_graph_chain(eng, moes, layer, T, reps, torch):
 
 
 def bench_config(eng, layer, copies, T, steps, warmup, torch):
-    """Another layer type (configs[3]: Q4_K gate/up + Q6_K down): the same
-    measurement over `copies` copies in HBM."""
+    """Another layer type (Q4_K gate/up + Q6_K down): the same measurement over `copies` copies in HBM."""
     moes = [eng.moe(layer) for _ in range(copies)]
     from biv_amd import synth
-    h = synth.make_tokens(1000 + T, T, offsets=T > 1)  # ~N(0,1) (configs[3])
+    h = synth.make_tokens(1000 + T, T, offsets=T > 1)  # ~N(0,1)
     h_dev = torch.from_numpy(h).cuda()
     out_dev = torch.empty_like(h_dev)
     for i in range(warmup):
@@ -243,7 +242,7 @@ BF_TRAFFIC = {"gate_up": 1470939136, "down": 931569664}
 
 
 def bench_bf16_stack(eng, T, n_layers, passes, torch):
-    """configs[4]: n_layers BF16 MoE layers resident in HBM, a T-token chunk
+    """n_layers BF16 MoE layers resident in HBM, a T-token chunk
     through all of them with the feed-forward half of Model::layer between
     (x += moe(rms_norm(x)), model.rs:788-790).  The layers are copies of one
     generated layer (distinct allocations, so every layer's weights come from
@@ -309,7 +308,7 @@ def bench_bf16_stack(eng, T, n_layers, passes, torch):
 def bench_dense(eng, copies, steps, warmup, torch, n_embd=4096, n_ff=12288):
     """The dense SwiGLU FFN of the qwen35 dense models (dense_ffn,
     model.rs:1118-1126) at a 9B-sized shape, Q8_0, T = 1 and 5, over `copies`
-    copies in HBM: a widening beside the MoE block, not a BASELINE config."""
+    copies in HBM."""
     from biv_amd import synth
     layer = synth.make_dense(9, n_embd=n_embd, n_ff=n_ff)
     dens = [eng.dense(layer) for _ in range(copies)]
@@ -366,7 +365,7 @@ def main():
     ap.add_argument("--sweep", default="1,40,512", help="other T values to report ('' for none)")
     ap.add_argument("--cpu-seconds", type=float, default=10.0, help="CPU baseline budget (0 to skip)")
     ap.add_argument("--configs", default="kquant,bf16,dense",
-                    help="other BASELINE configs to run: kquant (Q4_K/Q6_K at T=1, 2048), bf16 (the 40-layer BF16 "
+                    help="other configurations to run: kquant (Q4_K/Q6_K at T=1, 2048), bf16 (the 40-layer BF16 "
                          "stack at T=4096), dense (the qwen35 dense FFN, 4096 x 12288 Q8_0); '' for none")
     ap.add_argument("--bf16-layers", type=int, default=40)
     ap.add_argument("--graph-reps", type=int, default=50,
@@ -447,7 +446,7 @@ def main():
         "vs_baseline": None,
         "dtype": "int8",
         "data": "synthetic (seeded N(0,0.02) weights quantised to Q8_0, N(0,1) tokens)",
-        "config": {"workload": "qwen35moe MoE FFN layer, Q8_0, decode-verify T=5 (configs[1])",
+        "config": {"workload": "qwen35moe MoE FFN layer, Q8_0, decode-verify T=5",
                    "n_embd": E, "n_expert": NE, "k": K, "n_ff": FF, "n_ff_shared": FF, "T": args.T,
                    "distinct_experts_U": main_res["U"], "layers_rotated": args.layers},
         "roofline": main_res["roofline"],

@@ -643,9 +643,10 @@ int forward(biv_hip_ctx *ctx, const biv_hip_moe *m, const float *h, int T, float
     // pairs per slot: decode keeps an expert's tokens together; larger passes
     // cut them so that hot experts and the shared expert spread over the GPU
     // (a matrix-core workgroup takes a whole slot: 256 BF16 pairs, 16 Q8_0)
-    // quantised matrices at prefill sizes run on the int8 matrix cores: gate/up
-    // when gate and up are Q8_0 or Q4_K (each pair of one type, routed and
-    // shared), down when the routed and shared down matrices are Q8_0 or Q6_K
+    // quantised matrices at prefill sizes run on the matrix cores: gate/up (f16
+    // word dots) when gate and up are Q8_0 or Q4_K (each pair of one type,
+    // routed and shared), down (int8 block dots) when the routed and shared
+    // down matrices are Q8_0 or Q6_K
     auto gu_ok = [](int g, int u) { return g == u && (g == biv::T_Q8_0 || g == biv::T_Q4K); };
     const bool mq_gu = T >= MFMA_MIN_T && gu_ok(m->gate->m.ty, m->up->m.ty) &&
                        (!has_shared || gu_ok(m->sg->m.ty, m->su->m.ty));
@@ -761,7 +762,7 @@ int forward(biv_hip_ctx *ctx, const biv_hip_moe *m, const float *h, int T, float
         } else if (mq_gu) {
             a.sh_chunk = biv::MFMA_Q8_TILE;
             a.xq = ra.xq;
-            HIP_TRY(ctx, biv::launch_mfma_gateup_exact(a, st), "expert gate/up (int8 mfma)");
+            HIP_TRY(ctx, biv::launch_mfma_gateup_exact(a, st), "expert gate/up (exact mfma)");
         } else {
             HIP_TRY(ctx, biv::launch_gateup(a, st), "expert gate/up");
         }

@@ -211,13 +211,13 @@ hipError_t launch_split_bf16(const float *x, int rows, int K, void *xh, void *xl
 hipError_t launch_mfma_gateup(const MfArgs &a, hipStream_t st);
 hipError_t launch_mfma_down(const MfArgs &a, hipStream_t st);
 
-// Quantised experts at prefill sizes on the int8 matrix cores (mfma.hip),
-// with the chain kernels' contract (MvArgs: Q8 input rows a.xq / a.xd / a.xs,
-// f32 out, dump taps) and slots of at most MFMA_Q8_TILE pairs.  gate/up
-// (exact.hip; Q8_0 or Q4_K, gate and up of one type; the Q8 rows in
-// launch_quant_f16's order): bit for bit the x86 order.  down (Q8_0 or Q6_K):
-// exact int32 block dots (Q6_K: 16-element halves times their sub-scales),
-// f32 sums over blocks in an order of their own.
+// Quantised experts at prefill sizes on the matrix cores, with the chain
+// kernels' contract (MvArgs: Q8 input rows a.xq / a.xd / a.xs, f32 out, dump
+// taps) and slots of at most MFMA_Q8_TILE pairs.  gate/up (exact.hip, f16
+// MFMAs; Q8_0 or Q4_K, gate and up of one type; the Q8 rows in
+// launch_quant_f16's order): bit for bit the x86 order.  down (mfma.hip, int8
+// MFMAs; Q8_0 or Q6_K): exact int32 block dots (Q6_K: 16-element halves times
+// their sub-scales), f32 sums over blocks in an order of their own.
 constexpr int MFMA_Q8_TILE = 16;
 hipError_t launch_mfma_gateup_exact(const MvArgs &a, hipStream_t st);
 hipError_t launch_q8_mfma_down(const MvArgs &a, hipStream_t st);

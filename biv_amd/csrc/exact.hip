@@ -167,10 +167,11 @@ template <int TY, int NT> struct ExLds {
     static constexpr int BYTES = 2 * BUF > EX ? 2 * BUF : EX;
 };
 template <int TY, int NT> constexpr int ex_halves() { return TY == T_Q8_0 && NT > 2 ? 2 : 1; }
-// waves per SIMD the registers allow
+// waves per SIMD the registers allow (the 64-row instances at all 256, with 1
+// of Q8_0, 11 of Q4_K and 5 of Q6_K spilled)
 template <int TY, int NT> constexpr int ex_waves() { return NT > 2 ? 2 : NT == 1 ? 4 : TY == T_Q8_0 ? 3 : 2; }
 
-// out[t][r] = row_r . x_t over rows of any multiple of 256 elements (dense
+// out[t][r] = row_r . x_t over rows of any multiple of 512 elements (dense
 // FFN): GATEUP silu(gate_r . x_t) * (up_r . x_t).  A workgroup takes up to 16
 // NTM input rows and 16 output rows of gate and up (waves: gate, up x the two
 // parities), or 32 output rows (two 16-row tiles x the two parities); input
@@ -443,6 +444,10 @@ __global__ __launch_bounds__(EX_NTH) __attribute__((amdgpu_waves_per_eu(ex_waves
 // elements; Q4_K, whose bytes hold both parities, two of four).  A wave holds
 // both matrices' chains of the 16 pairs (128 accumulators), so the tree and
 // the SwiGLU need no exchange between lanes.
+//
+// DUMP: the instance that writes the integer block dots, for the taps only (it
+// spills 530 to 730 VGPRs; the f32 chains that matter are the other's, which
+// the block's outputs test).
 constexpr int GS_WAVES = 4;
 constexpr int GS_NTH = 64 * GS_WAVES;
 constexpr int GS_ROWS = MFMA_Q8_TILE;       // pairs of a slot

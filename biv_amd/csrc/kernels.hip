@@ -296,7 +296,7 @@ __device__ inline void quant_quad(const float (&v)[8], int E, int t, int b, int 
 // What a k_router instance does before the logits: nothing, or the post_norm
 // (norm_w), for few tokens or many; and whether h is quantised as f16 (F16).
 // Compiled apart: in one kernel the few-token norm's registers were every
-// caller's (2048 wide, 256 threads: 140 VGPRs, 3 waves a SIMD, against 95 and 5
+// caller's (2048 wide, 256 threads: 140 VGPRs, 3 waves a SIMD, against 69 and 7
 // without it; layers of 64 experts at 2 to 16 tokens 0.5-0.9% slower, the step
 // at 17 and 40 tokens 1%, at 1 token 16.9 against 16.4 us).
 enum { NORM_NONE, NORM_FEW, NORM_MANY };

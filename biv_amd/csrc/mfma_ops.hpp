@@ -76,12 +76,5 @@ __device__ __forceinline__ uint2 i8x4_to_f16x4(uint32_t q) { return bytes_to_f16
 
 __device__ inline float f16_to_f32(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
 
-// byte i (0..15) of a 16-byte vector
-__device__ inline int byte_at4(const int4 &v, int i)
-{
-    const int w = i < 4 ? v.x : i < 8 ? v.y : i < 12 ? v.z : v.w;
-    return ((unsigned)w >> (8 * (i & 3))) & 0xFF;
-}
-
 } // namespace
 } // namespace biv

@@ -7,7 +7,7 @@
    chains of 1368-1382).  The intermediate is quantised again before down, and
    a value that lands on the other side of a rounding boundary moves a quant
    by one step: at the Q8_0 T = 512 Zipf config this alone moves the layer's
-   output past the north star's bar of 1e-3 * RMS.
+   output past the bar of 1e-3 * RMS.
 
 2. The BF16 grouped GEMM multiplies the weights by both bf16 halves of the
    f32 activations (hi = bf16(x), lo = bf16(x - hi)).  Dropping the lo half of

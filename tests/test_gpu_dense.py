@@ -4,7 +4,7 @@ dense_ffn, model.rs:1118-1126) on the GPU with the CPU oracle's dense_ffn.
 The rows of a dense FFN are longer than the experts' (n_ff up to 17408 in
 the qwen35 dense models), so the kernels stream each row in chunks of 512
 elements and carry the reference's 16 x86 chains across the chunks: every
-output carries the oracle's bits (the bar asserted is the north star's
+output carries the oracle's bits (the bar asserted is
 max|d| <= 1e-3 * RMS plus >= 99.99% identical bits).
 """
 import numpy as np

@@ -41,7 +41,7 @@ def layer_for(engine, **kw):
 
 
 def check_output(ref, got, tol=TOL, min_exact=0.9999):
-    """max|d| <= tol * RMS (the north star's bar); and, since every sum runs
+    """max|d| <= tol * RMS (the bar); and, since every sum runs
     in the reference's order and exp is glibc's to the bit, the outputs carry
     the reference's exact bits (measured: all of them; the bar leaves room for
     the 2 in 2.2e9 inputs where the restated expf is one ulp off)."""
@@ -146,9 +146,10 @@ def test_q8_small_layer(orc, engine, T):
     """T <= 16 quantises the SwiGLU intermediate inside the down kernel,
     larger T in its own launch; below 64 every sum runs in the x86 order and
     the outputs carry the oracle's bits.  From T = 64 the experts run on the
-    int8 matrix cores (slots of 16 pairs): the int32 block dots are still the
-    oracle's exactly (checked from the MFMA kernel's own taps), the f32 sums
-    over blocks run in another order, so the outputs meet the tolerance.
+    matrix cores (slots of 16 pairs): the int32 block dots are still the
+    oracle's exactly (checked from the kernels' taps; gate/up with taps is an
+    instance of its own, whose output the one without has to equal), down's f32 sums over blocks run in another order, so the outputs
+    meet the tolerance.
     Each side of every switch: 16/17 (down + combine in one launch), 63/64
     (chain kernels / matrix cores), 255/256 (decode router / pre-pass and
     matrix-core router), 512/513 (the dispatch scan inside the placement /
@@ -459,8 +460,8 @@ def test_bf16_layer(orc, engine, T):
 @pytest.mark.parametrize("T,n_expert", [(64, 32), (255, 32), (256, 32), (300, 32), (512, 256)])
 def test_bf16_mfma(orc, engine, T, n_expert):
     """BF16 experts from T = 64 on the matrix cores: activations split into
-    two bf16 halves, products exact, sums in the MFMA's order.  The bar is the
-    north star's max|d| <= 1e-3 * RMS; routing (the f32 router) stays exact."""
+    two bf16 halves, products exact, sums in the MFMA's order.  The bar is
+    max|d| <= 1e-3 * RMS; routing (the f32 router) stays exact."""
     print(f"case bf16 mfma T={T} experts={n_expert}", flush=True)
     layer, moe = layer_for(engine, seed=83, n_expert=n_expert, types=(BF16, BF16, BF16))
     h = synth.make_tokens(800 + T, T, offsets=True)
@@ -497,9 +498,9 @@ def test_rms_norm(orc, engine, n):
 def test_q8_ffn_step(orc, engine, T):
     """The FFN half of Model::layer on a Q8_0 layer (model.rs:786-790):
     x += moe(rms_norm(x, post_norm)).  Below 256 tokens the router launch
-    forms the norm itself (its workgroups normalise the staged rows, the
-    quantising ones write the normalised rows); from 256 a norm launch runs
-    first.  Full-size layer (256 experts); T = 512 with Zipf-skewed routing."""
+    forms the norm itself (at 1 and 5 tokens its row workgroups normalise as
+    they read, the quantising ones write the normalised rows); from 256 the
+    pre-pass does.  Full-size layer (256 experts); T = 512 with Zipf-skewed routing."""
     print(f"case q8 ffn_step T={T}", flush=True)
     layer, moe = layer_for(engine, seed=1)
     E, eps = layer.n_embd, 1e-6
@@ -555,7 +556,7 @@ def test_bf16_stack_steps(orc, engine):
 
 
 def test_bf16_stack_depth_40(orc, engine):
-    """configs[4]'s depth: x += moe(rms_norm(x)) through 40 applications of a
+    """A 40-layer stack's depth: x += moe(rms_norm(x)) through 40 applications of a
     256-expert BF16 layer (each with its own norm weights), a T = 64 chunk on
     the matrix-core path, against the oracle after every layer: the error the
     bf16 halves' own summation order leaves must not grow past the bar over
@@ -598,10 +599,12 @@ def test_kquant_layer(orc, engine):
 
 @pytest.mark.parametrize("T", [64, 100, 255, 256])
 def test_kquant_prefill(orc, engine, T):
-    """From T = 64 the K-quant experts run on the int8 matrix cores: Q4_K
-    gate/up bit for bit (word dots from masked MFMAs, the x86 chains and the
-    mins on the vector ALU), Q6_K down with exact block int32s (each 16-element
-    half times its sub-scale) summed in another order."""
+    """From T = 64 the K-quant experts run on the matrix cores: Q4_K gate/up bit
+    for bit (word dots and scale products from f16 and f32 MFMAs, the x86 chains
+    on the vector ALU), Q6_K down with exact block int32s (each 16-element half
+    times its sub-scale) summed in another order.  The block dots are
+    the kernels' taps; gate/up with taps is an instance of its own, whose output
+    the one without has to equal."""
     print(f"case kquant prefill T={T}", flush=True)
     layer, moe = layer_for(engine, seed=31, n_expert=32, types=(Q4K, Q4K, Q6K))
     h = synth.make_tokens(400 + T, T, offsets=True)
@@ -626,7 +629,7 @@ def _full_size(orc, moe, layer, h, exact_ids=True, dots_sample=0):
 
 
 def test_kquant_full_size_2048(orc, engine):
-    """configs[3] at its full size: 256 experts, Q4_K gate/up and Q6_K down,
+    """The Q4_K/Q6_K layer at its full size: 256 experts, Q4_K gate/up and Q6_K down,
     T = 2048 (the matrix-core kernels, exact Q4_K gate/up)."""
     print("case kquant full T=2048", flush=True)
     layer, moe = layer_for(engine, seed=33, types=(Q4K, Q4K, Q6K))
@@ -636,7 +639,7 @@ def test_kquant_full_size_2048(orc, engine):
 
 
 def test_kquant_full_size_decode(orc, engine):
-    """configs[3] at T = 1 and 5 with its full 256-expert router: the chain
+    """The same at T = 1 and 5 with the full 256-expert router: the chain
     kernels, bit-identical to the oracle."""
     layer, moe = layer_for(engine, seed=33, types=(Q4K, Q4K, Q6K))
     for T in (1, 5):
@@ -645,7 +648,7 @@ def test_kquant_full_size_decode(orc, engine):
 
 
 def test_bf16_stack_full_size(orc, engine):
-    """configs[4]'s step at its full size: x += moe(rms_norm(x)) through two
+    """The BF16 step at its full size: x += moe(rms_norm(x)) through two
     256-expert BF16 layers with a T = 4096 chunk (the pre-pass forms the
     post_norm, the matrix-core router, the bf16 grouped GEMMs), against the
     oracle after each layer (tolerance: the bf16 halves sum in their own
@@ -676,7 +679,7 @@ def test_bf16_stack_full_size(orc, engine):
 
 
 def test_bf16_full_size_4096(orc, engine):
-    """configs[4]'s layer at its full size: 256 BF16 experts, T = 4096 (bf16
+    """The BF16 layer at its full size: 256 experts, T = 4096 (bf16
     MFMA grouped GEMM on hi/lo halves of the f32 activations)."""
     print("case bf16 full T=4096", flush=True)
     layer, moe = layer_for(engine, seed=2, types=(BF16, BF16, BF16))
