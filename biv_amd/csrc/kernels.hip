@@ -253,9 +253,14 @@ __device__ inline float rms_scale(float acc, int n, float eps)
     return 1.0f / sqrtf(ss + eps);
 }
 
-// tokens up to which the router launch's post_norm and quantisation take a
-// wave per 16 blocks (past it there are waves enough with a half wave a token)
-constexpr int ROUTER_FEW_T = 16;
+// Tokens up to which the router launch's post_norm and quantisation take a
+// wave per 16 blocks.  Against a half wave a token, the step through 4 layers of
+// 64 experts, 2048 wide: 9 / 16 / 17 / 33 / 63 tokens 202 / 256 / 262 / 328 /
+// 471 against 225 / 278 / 280 / 345 / 486 us (1024 wide at 16 tokens 222 against
+// 231, 512 wide 194 against 198, alike past 16).  Past it there are waves enough
+// with the half waves (2 BF16 layers at 65 / 100 / 255 tokens 364 / 380 / 428 us
+// against 364 / 382 / 430 with a wave per 16 blocks).
+constexpr int ROUTER_FEW_T = 64;
 
 // lane x's value from the lane next to it (x ^ 1), or two on (x ^ 2), of its four
 __device__ inline float quad_xor1(float x) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, true)); }
@@ -3010,8 +3015,8 @@ hipError_t launch_router(const RouterArgs &a0, hipStream_t st)
         if (a.f16 && a.T <= 64) return launch_router_n<NS, TC / 2, NORM_MANY, true>(a, st);                     \
         if (a.f16) return launch_router_n<NS, 2 * TC, NORM_MANY, true>(a, st);                                  \
         if (a.T == 1) return launch_router_n<NS, TC, NORM_FEW, false, ROUTER_T1_NTH>(a, st);                    \
-        if (a.T <= ROUTER_FEW_T) return launch_router_n<NS, TC / 4, NORM_FEW, false>(a, st);                    \
-        if (a.T <= 64) return launch_router_n<NS, TC / 2, NORM_MANY, false>(a, st);                             \
+        if (a.T <= 16) return launch_router_n<NS, TC / 4, NORM_FEW, false>(a, st);                              \
+        if (a.T <= ROUTER_FEW_T) return launch_router_n<NS, TC / 2, NORM_FEW, false>(a, st);                    \
         return launch_router_n<NS, 2 * TC, NORM_MANY, false>(a, st);                                            \
     }
     BIV_ROUTER_CASE(64)

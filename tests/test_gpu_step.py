@@ -1,6 +1,7 @@
 """biv_hip_moe_ffn_step, x += moe(rms_norm(x)), against the oracle at every
-width: on both sides of the router launch's switch at 16/17 tokens, and with
-the f16 quants of 64 tokens and up, to 256, where the pre-pass takes over.
+width: on both sides of the router launch's switches at 16/17 and 64/65 tokens,
+and with the f16 quants of 64 tokens and up, to 256, where the pre-pass takes
+over.
 Every sum runs in the reference's order (from 64 tokens with a Q4_K down, which
 stays on the chain kernels), so the bound is equality."""
 import numpy as np
@@ -71,7 +72,14 @@ def against_oracle(orc, engine, layer, n_embd, tokens):
 @pytest.mark.parametrize("shared", [True, False])
 def test_step_few_tokens(orc, engine, n_embd, types, shared):
     layer = synth.make_layer(42, n_embd=n_embd, n_expert=20, k=4, types=types, shared=shared)
-    against_oracle(orc, engine, layer, n_embd, (1, 2, 3, 4, 6, 15, 16, 17, 33))
+    against_oracle(orc, engine, layer, n_embd, (1, 2, 3, 4, 6, 15, 16, 17, 33, 63))
+
+
+# Q6_K gate/up, which stays on the chain kernels: no f16 quants
+@pytest.mark.parametrize("n_embd", [512, 1024, 2048])
+def test_step_chains(orc, engine, n_embd):
+    layer = synth.make_layer(44, n_embd=n_embd, n_expert=20, k=4, types=(Q6K, Q6K, Q4K))
+    against_oracle(orc, engine, layer, n_embd, (64, 65, 255, 256))
 
 
 @pytest.mark.parametrize("n_embd", [512, 1024, 2048])
