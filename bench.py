@@ -68,7 +68,7 @@ TRAFFIC_SOURCE = "profiles/moe_layer_q8_0_hbm_traffic.md (rocprofv3 --pmc FETCH_
 TRAFFIC = {
     ("gate_up", 1): 20207131, ("gate_up", 5): 91705677, ("gate_up", 40): 430113924,
     ("down", 1): 10344203, ("down", 5): 46907741, ("down", 40): 217679560,
-    ("down", 512): 365848576,
+    ("gate_up", 512): 685275136, ("down", 512): 365893632,
 }
 
 
@@ -231,13 +231,13 @@ def bench_config(eng, layer, copies, T, steps, warmup, torch):
                            "achieved": round(ach / 1e9, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                            "frac": round(ach / HBM_PEAK, 4), "bytes_per_launch": gbytes, "avg_us": round(kern_us, 3),
                            "traffic": KQ_TRAFFIC.get("gate_up"),
-                           "traffic_source": KQ_TRAFFIC_SOURCE if "gate_up" in KQ_TRAFFIC else None}
+                           "traffic_source": KQ_TRAFFIC_SOURCE}
     return res
 
 
 # as TRAFFIC, for the Q4_K/Q6_K layer at T = 2048 and the BF16 layer at T = 4096
 KQ_TRAFFIC_SOURCE = "profiles/prefill_hbm_traffic.md (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE; copy-calibrated)"
-KQ_TRAFFIC = {"down": 585138176}
+KQ_TRAFFIC = {"gate_up": 702646272, "down": 585138176}
 BF_TRAFFIC = {"gate_up": 1470939136, "down": 931569664}
 
 
